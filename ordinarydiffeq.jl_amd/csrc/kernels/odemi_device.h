@@ -129,12 +129,14 @@ template <typename T>
 __device__ __forceinline__ T max_fast(T x, T y) { return y > x ? y : x; }
 
 // FP64 reciprocal, quotient and square root from the hardware estimates
-// (v_rcp_f64, v_rsq_f64) with Newton-Raphson refinement: FP64-accurate to about
-// one ulp but not always the correctly rounded result.  The mixed-precision
-// lane engine's error norm and controller use them (FP64 range and precision
-// without the IEEE division and square-root sequences); the FP64 engines keep
-// IEEE / and sqrt for bit parity with the CPU restatement.  Positive normal
-// operands (tolerance-scaled denominators, step-size ratios).
+// (v_rcp_f64, v_rsq_f64) refined by fma steps: the estimate's Newton steps, then
+// one residual correction of the quotient (two of the root).  While no
+// intermediate over- or underflows these are the correctly rounded results
+// (Markstein's method), so an operand range check replaces the scaling and
+// fix-up instructions of the IEEE forms: 8 instructions for a quotient against
+// 11, 3 with a constant divisor.  The step loops use them where they have
+// checked the range (tsit5_attempt_fast, rodas_attempt_fast), the mixed engines
+// throughout; elsewhere the FP64 engines use / and sqrt.
 __device__ __forceinline__ double rcp_nr(double b) {
     double r = __builtin_amdgcn_rcp(b);
     double e = fma(-b, r, 1.0);
@@ -142,21 +144,33 @@ __device__ __forceinline__ double rcp_nr(double b) {
     e = fma(-b, r, 1.0);
     return fma(r, e, r);
 }
-__device__ __forceinline__ double div_nr(double a, double b) {
-    const double r = rcp_nr(b);
+// a / b with r = rcp_nr(b)
+__device__ __forceinline__ double div_by_rcp(double a, double b, double r) {
     const double q = a * r;
     return fma(fma(-b, q, a), r, q);
 }
-__device__ __forceinline__ double sqrt_nr(double x) {   // x >= 0
-    const bool tiny = x < 0x1p-1000;                       // keep the estimate off subnormals
-    const double xs = tiny ? x * 0x1p+1000 : x;
-    const double y = __builtin_amdgcn_rsq(xs);
-    double g = xs * y, h = 0.5 * y;
-    const double r = fma(-g, h, 0.5);
+__device__ __forceinline__ double div_nr(double a, double b) { return div_by_rcp(a, b, rcp_nr(b)); }
+// a / b for two values of FP32 precision (24 significant bits each): the
+// quotient is at least 2^-78 (relative) away from any rounding boundary, so one
+// Newton step before the exact residual is enough.
+__device__ __forceinline__ double div_f32_values(double a, double b) {
+    double r = __builtin_amdgcn_rcp(b);
+    r = fma(r, fma(-b, r, 1.0), r);
+    return div_by_rcp(a, b, r);
+}
+// sqrt(x) for 2^-700 <= x < 2^1000
+__device__ __forceinline__ double sqrt_inrange(double x) {
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double r = fma(-h, g, 0.5);
     g = fma(g, r, g);
     h = fma(h, r, h);
-    g = fma(fma(-g, g, xs), h, g);
-    g = fma(fma(-g, g, xs), h, g);
+    g = fma(fma(-g, g, x), h, g);
+    return fma(fma(-g, g, x), h, g);
+}
+__device__ __forceinline__ double sqrt_nr(double x) {   // x >= 0
+    const bool tiny = x < 0x1p-1000;                       // keep the estimate off subnormals
+    double g = sqrt_inrange(tiny ? x * 0x1p+1000 : x);
     g = tiny ? g * 0x1p-500 : g;
     return (x > 0.0 && x < __builtin_huge_val()) ? g : x;   // 0, inf, NaN pass through
 }
@@ -215,39 +229,49 @@ __device__ __forceinline__ double det_exp(double x) {
 constexpr double kLN10 = 2.302585092994046, kLN2 = 0.6931471805599453;
 
 // FastPower.jl 1.1.x `fastpower` (controllers.jl:815-816): Goldberg's rational
-// fast log2 in Float32, then exp2 of the Float32 product evaluated in double
-// (det_exp) and rounded once to Float32.
+// fast log2 in Float32, then exp2 of the Float32 product, rounded once to
+// Float32.  The significand after the select lies in [-1/2, 1/2), so the
+// rational's quotient needs no scaling: v_rcp_f32, one Newton step and one
+// residual correction give the IEEE quotient for each of the 2^24 significands.
 __device__ __forceinline__ float fastlog2f(float x) {
-    unsigned ux1i = __float_as_uint(x);
-    unsigned ex = (ux1i & 0x7F800000u) >> 23;
-    float signif, fexp;
-    if ((ux1i & 0x00400000u) != 0u) {
-        signif = __uint_as_float((ux1i & 0x007FFFFFu) | 0x3f000000u);
-        fexp = (float)ex - 126.0f;
-    } else {
-        signif = __uint_as_float((ux1i & 0x007FFFFFu) | 0x3f800000u);
-        fexp = (float)ex - 127.0f;
-    }
-    signif = signif - 1.0f;
-    float t1 = 0.338953f * signif;
-    float t2 = t1 + 2.198599f;
-    float t3 = signif * t2;
-    float t4 = signif + 1.523692f;
-    float t5 = t3 / t4;
+    const unsigned ux1i = __float_as_uint(x);
+    const unsigned ex = (ux1i & 0x7F800000u) >> 23;
+    const bool hi = (ux1i & 0x00400000u) != 0u;
+    const float signif = __uint_as_float((ux1i & 0x007FFFFFu) | (hi ? 0x3f000000u : 0x3f800000u)) - 1.0f;
+    const float fexp = (float)ex - (hi ? 126.0f : 127.0f);
+    const float t3 = signif * (0.338953f * signif + 2.198599f);
+    const float t4 = signif + 1.523692f;
+    float r = __builtin_amdgcn_rcpf(t4);
+    r = fmaf(r, fmaf(-t4, r, 1.0f), r);
+    float t5 = t3 * r;
+    t5 = fmaf(fmaf(-t4, t5, t3), r, t5);
     return fexp + t5;
 }
-__device__ __forceinline__ double fastpower(double x, double y) {
-    if (x == 0.0) return 0.0;
-    if (isinf(x) && isinf(y)) return __longlong_as_double(0x7ff0000000000000LL);
-    float lg = fastlog2f((float)x);
-    float prod = (float)y * lg;
-    return (double)(float)det_exp((double)prod * kLN2);
+// exp2 of a Float32 value rounded once to Float32: 2^rint(p) times a degree-10
+// polynomial for 2^f, |f| <= 1/2, in FP64 (fitted on Chebyshev nodes to 9e-16).
+// It returns the same Float32 as (float)det_exp(p ln 2), the restatement's form,
+// for every Float32 |p| <= 30 (all 2.2e9 of them compared), at 14 instructions
+// instead of ~45 (det_exp divides).  The controllers' |p| stays below 21.
+__device__ __forceinline__ float exp2_f32(float p) {
+    const float k = __builtin_rintf(p);
+    const double f = (double)(p - k);
+    double a = 0x1.e5e9f548e5725p-28;
+    a = fma(a, f, 0x1.b6571de2f2351p-24);
+    a = fma(a, f, 0x1.62bfe46117445p-20);
+    a = fma(a, f, 0x1.ffcb76789860fp-17);
+    a = fma(a, f, 0x1.4309130378460p-13);
+    a = fma(a, f, 0x1.5d87fe908f88ap-10);
+    a = fma(a, f, 0x1.3b2ab6fba385fp-7);
+    a = fma(a, f, 0x1.c6b08d7044119p-5);
+    a = fma(a, f, 0x1.ebfbdff82c590p-3);
+    a = fma(a, f, 0x1.62e42fefa39f7p-1);
+    a = fma(a, f, 1.0);
+    return __builtin_ldexpf((float)a, (int)k);
 }
-// The same fastpower with the hardware reciprocal in Goldberg's rational and
-// the hardware exp2 (v_rcp_f32 / v_exp_f32, ~1 ulp): the mixed-precision lane
-// engines' controller.  FastPower evaluates exp2 under @fastmath; this form is
-// not bit-matched to the CPU restatement (those engines are checked to
-// tolerance).
+// The mixed-precision lane engines' forms with the hardware reciprocal and exp2
+// (v_rcp_f32 / v_exp_f32, ~1 ulp).  FastPower evaluates exp2 under @fastmath;
+// these are not bit-matched to the CPU restatement (those engines are checked
+// to tolerance).
 __device__ __forceinline__ float fastlog2_hw(double x) {
     const float xf = (float)x;
     const unsigned ux = __float_as_uint(xf);
@@ -258,10 +282,16 @@ __device__ __forceinline__ float fastlog2_hw(double x) {
     const float t3 = signif * (0.338953f * signif + 2.198599f);
     return fexp + t3 * __builtin_amdgcn_rcpf(signif + 1.523692f);
 }
-__device__ __forceinline__ float fastpower_hw(double x, double y) {
-    if (x == 0.0) return 0.0f;
-    if (isinf(x) && isinf(y)) return __builtin_huge_valf();
-    return __builtin_amdgcn_exp2f((float)y * fastlog2_hw(x));
+// fastpower(x, y) = pow_of_log2(y, log2 x) in either form
+template <bool HW>
+__device__ __forceinline__ float fast_log2(double x) {
+    if constexpr (HW) return fastlog2_hw(x);
+    else return fastlog2f((float)x);
+}
+template <bool HW>
+__device__ __forceinline__ float pow_of_log2(double y, float lg) {
+    if constexpr (HW) return __builtin_amdgcn_exp2f((float)y * lg);
+    else return exp2_f32((float)y * lg);
 }
 
 // ---------------------------------------------------------------------------
@@ -344,7 +374,7 @@ __constant__ double kRH[3][8] = {
 // Common per-trajectory controller / loop state (all FP64)
 // ---------------------------------------------------------------------------
 struct Ctl {
-    double t, dt, dtpropose, tprev, tf, dtmax, EEst, q11, errold;
+    double t, dt, dtpropose, tprev, tf, dtmax, EEst, q11;
     double tdir;   // integration direction sign(tf - t0) (+1 when tf == t0); dt and dtmax carry it
     int iter, success_iter, accept_step, next_step_tstop;
     int isout;   // the last attempt's isoutofdomain verdict (integrator.isout)
@@ -364,8 +394,8 @@ struct Ctl {
     int event_last;
     unsigned sim_mask;   // its components when a vector callback's (prev_simultaneous_events)
     double last_event_error;
-    // mixed engines: fastpower(errold, beta2), kept from the accept that set
-    // errold (NaN: not known yet), and log2(EEst) of the last controller call
+    // fastpower(errold, beta2), kept from the accept that set errold in place of
+    // errold itself, and log2(EEst) of the last controller call
     float erroldp, lgEEst;
 };
 
@@ -415,8 +445,17 @@ __device__ __forceinline__ void fix_dt_at_bounds(Ctl& c, double dtmin) {
         c.dt = jl_min(c.dt, dmin);
     }
 }
+// fastpower(errold, beta2) of the initial errold = qoldinit
+template <bool HW>
+__device__ __forceinline__ float erroldp_init() {
+    double x = 1e-4;
+    if constexpr (HW) asm("" : "+v"(x));   // the hardware's estimates, not the compiler's folded ones
+    return pow_of_log2<HW>(0.08, fast_log2<HW>(x));
+}
+
 // controllers.jl:805-821.  HW: the mixed engine's form (FastPower's Float32
 // log2/exp2 with the hardware reciprocal and exp2, FP64 quotients by div_nr).
+// q11 and fastpower(errold, beta2) are Float32 values, q lies in [1e-6, 1e7].
 template <bool HW = false>
 __device__ __forceinline__ double stepsize_controller(Ctl& c, const CtlConst& k) {
     // 1/qmax as a select of two folded constants, not a division per attempt
@@ -425,19 +464,13 @@ __device__ __forceinline__ double stepsize_controller(Ctl& c, const CtlConst& k)
     if (c.EEst == 0.0) {
         q = lo;
     } else {
-        double q11, x;
-        if constexpr (HW) {
-            // fastpower_hw(EEst, beta1) with its log2 kept for the accept;
-            // errold's power comes from the accept that set it
-            c.lgEEst = fastlog2_hw(c.EEst);
-            q11 = __builtin_amdgcn_exp2f((float)k.beta1 * c.lgEEst);
-            if (c.erroldp != c.erroldp) c.erroldp = fastpower_hw(c.errold, k.beta2);
-            x = div_nr(q11, (double)c.erroldp * k.gamma);
-        } else {
-            q11 = fastpower(c.EEst, k.beta1);
-            q = q11 / fastpower(c.errold, k.beta2);
-            x = q / k.gamma;
-        }
+        // log2(EEst) is kept for the accept; errold's power comes from the accept
+        // that set it
+        double x;
+        c.lgEEst = fast_log2<HW>(c.EEst);
+        const double q11 = pow_of_log2<HW>(k.beta1, c.lgEEst);
+        if constexpr (HW) x = div_nr(q11, (double)c.erroldp * k.gamma);
+        else x = div_f32_values(q11, c.erroldp) / k.gamma;
         c.q11 = q11;
         q = (x > hi) ? hi : ((x < lo) ? lo : x);
     }
@@ -447,25 +480,24 @@ __device__ __forceinline__ double stepsize_controller(Ctl& c, const CtlConst& k)
 template <bool HW = false>
 __device__ __forceinline__ void accept_controller(Ctl& c, const CtlConst& k, double q, double dtmin) {
     if (k.qsteady_min <= q && q <= k.qsteady_max) q = 1.0;
-    c.errold = jl_max(c.EEst, k.qoldinit);
+    // errold = max(EEst, qoldinit): above qoldinit its power comes from the log2
+    // that the controller took of EEst
+    c.erroldp = (c.EEst > k.qoldinit) ? pow_of_log2<HW>(k.beta2, c.lgEEst) : erroldp_init<HW>();
     double dtnew;
-    if constexpr (HW) {
-        // errold = EEst (nonzero: the controller took its log2) gives
-        // fastpower_hw(errold, beta2) from that log2, bit for bit
-        c.erroldp = (c.errold == c.EEst) ? __builtin_amdgcn_exp2f((float)k.beta2 * c.lgEEst)
-                                         : fastpower_hw(c.errold, k.beta2);
-        dtnew = div_nr(c.dt, q);   // q in [1/qmax, 1/qmin]
-    } else {
-        dtnew = c.dt / q;
-    }
+    if constexpr (HW) dtnew = div_nr(c.dt, q);   // q in [1/qmax, 1/qmin]
+    else dtnew = c.dt / q;
     double dp = c.tdir * jl_min(fabs(c.dtmax), fabs(dtnew));
     c.dtpropose = c.tdir * jl_max(fabs(dp), fabs(jl_max(jl_eps(c.t), dtmin)));
 }
-// controllers.jl:838-843 (HW: the mixed engines' Newton-refined FP64 quotients;
-// a wave runs this whenever any of its lanes rejects, i.e. nearly every attempt)
+// The next attempt's dt after a rejection: step_reject_controller!
+// (controllers.jl:838-843), or dt * qmin when isoutofdomain flagged the step
+// (handle_step_rejection!, integrator_utils.jl:135-136).  The reference runs it
+// in the next loop header; here it ends the rejected attempt (dt is not read in
+// between), so no controller value but erroldp outlives an attempt.
 template <bool HW = false>
 __device__ __forceinline__ void reject_controller(Ctl& c, const CtlConst& k) {
-    if constexpr (HW) c.dt = div_nr(c.dt, jl_min(1.0 / k.qmin, div_nr(c.q11, k.gamma)));
+    if (c.isout) c.dt = c.dt * k.qmin;
+    else if constexpr (HW) c.dt = div_nr(c.dt, jl_min(1.0 / k.qmin, div_nr(c.q11, k.gamma)));
     else c.dt = c.dt / jl_min(1.0 / k.qmin, c.q11 / k.gamma);
 }
 
@@ -687,15 +719,17 @@ __device__ __forceinline__ double user_dt(const Ctl& c, const Params& P) {
 }
 
 // Common per-trajectory initialisation of the controller state.
-__device__ __forceinline__ void ctl_init_t(Ctl& c, const Params& P, double t0, double tf) {
+// hw: the mixed lane engines' FastPower forms.
+__device__ __forceinline__ void ctl_init_t(Ctl& c, const Params& P, double t0, double tf, bool hw) {
     c.t = t0; c.tprev = t0; c.tf = tf;
     c.tdir = (tf < t0) ? -1.0 : 1.0;
     // dtmax defaults to tf - t0; a positive one takes tdir's sign (solve.jl:401)
     c.dtmax = (P.dtmax > 0.0) ? c.tdir * P.dtmax : (tf - t0);
-    c.EEst = 1.0; c.q11 = 1.0; c.errold = 1e-4;
+    c.EEst = 1.0; c.q11 = 1.0;
     c.iter = 0; c.success_iter = 0; c.accept_step = 0; c.next_step_tstop = 0; c.isout = 0;
     c.reeval_fsal = 0; c.ncond = 0; c.event_last = 0; c.sim_mask = 0u; c.last_event_error = 0.0;
-    c.erroldp = __builtin_nanf(""); c.lgEEst = 0.0f;
+    c.erroldp = hw ? erroldp_init<true>() : erroldp_init<false>();
+    c.lgEEst = 0.0f;
     c.dt = 0.0; c.dtpropose = 0.0;
     c.nf = 0; c.naccept = 0; c.nreject = 0; c.njacs = 0; c.nw = 0; c.nsolve = 0;
     c.nsaved = 0; c.spos = 0; c.send = 0; c.tf_in_saveat = 0;
@@ -703,7 +737,9 @@ __device__ __forceinline__ void ctl_init_t(Ctl& c, const Params& P, double t0, d
     c.tsp = 0; c.tsend = 0; c.tnext = tf;
     if (P.ntstops > 0) tstops_init(c, P, t0);
 }
-__device__ __forceinline__ void ctl_init(Ctl& c, const Params& P, i64 j) { ctl_init_t(c, P, P.t0[j], P.tf[j]); }
+__device__ __forceinline__ void ctl_init(Ctl& c, const Params& P, i64 j, bool hw = false) {
+    ctl_init_t(c, P, P.t0[j], P.tf[j], hw);
+}
 
 // solution_endpoint_match_cur_integrator! (integrator_utils.jl:540-588) and
 // result write-out.
@@ -807,7 +843,7 @@ struct Tsit5Lane {
 template <typename S, typename K, int N>
 __device__ __forceinline__ void tsit5_load(Tsit5Lane<S, K, N>& L, const Params& P, i64 j, double (&u0d)[N],
                                            double (&pd)[ODEMI_NP]) {
-    ctl_init(L.c, P, j);
+    ctl_init(L.c, P, j, sizeof(K) < sizeof(S));
 #pragma unroll
     for (int i = 0; i < N; i++) { u0d[i] = P.u0[(i64)i * P.N + j]; L.u[i] = (S)u0d[i]; L.uprev[i] = L.u[i]; }
 #pragma unroll
@@ -833,7 +869,7 @@ template <typename S, typename K, int N>
 __device__ __forceinline__ void tsit5_init(Tsit5Lane<S, K, N>& L, const Params& P, i64 j, i64 slot = -1) {
     if (P.rec_in) {   // the record prep wrote for this queue slot
         const double* r = P.rec_in + slot * rec_in_words(N, ODEMI_NP);
-        ctl_init_t(L.c, P, r[N + ODEMI_NP], r[N + ODEMI_NP + 1]);
+        ctl_init_t(L.c, P, r[N + ODEMI_NP], r[N + ODEMI_NP + 1], sizeof(K) < sizeof(S));
 #pragma unroll
         for (int i = 0; i < N; i++) { L.u[i] = (S)r[i]; L.uprev[i] = L.u[i]; }
 #pragma unroll
@@ -897,10 +933,11 @@ __device__ void tsit5_prep(const Params& P) {
 // and FP64 VALU ops issue at one rate, so the gain is in the operations dropped
 // (per-stage conversions, FastPower's exp2 through the exact FP64 det_exp, the
 // IEEE division and square-root fix-up sequences).
+// tsit5_stages: k2..k7, u and the embedded error sum (ea[i] = dt sum btilde_j kj)
+// of a step of size dt from (t, uprev, k1).
 template <typename S, typename K, int N>
-__device__ __forceinline__ void tsit5_perform_step_mixed(Tsit5Lane<S, K, N>& L, const Params& P) {
+__device__ __forceinline__ void tsit5_stages_mixed(Tsit5Lane<S, K, N>& L, double t, double dt, double (&ea)[N]) {
     typedef Tsit5Tab T;
-    const double t = L.c.t, dt = L.c.dt;
     const float dtf = (float)dt;
     float ub[N], e[N], tmp[N];
     const float a = (float)(dt * T::a21);
@@ -962,23 +999,18 @@ __device__ __forceinline__ void tsit5_perform_step_mixed(Tsit5Lane<S, K, N>& L, 
         tmp[i] = (float)L.u[i];
     }
     odemi_f<float>(L.k7, tmp, L.p, (float)(t + dt));
-    L.c.nf += 6;
-    double ea[N];   // utilde = dt * e, then the FP64 norm
 #pragma unroll
     for (int i = 0; i < N; i++) ea[i] = dt * (double)fmaf((float)T::bt7, L.k7[i], e[i]);
-    L.c.EEst = residual_norm_nr<N>(ea, L.uprev, L.u, P.abstol, P.reltol);
 }
 
 template <typename S, typename K, int N>
-__device__ __forceinline__ void tsit5_perform_step(Tsit5Lane<S, K, N>& L, const Params& P) {
+__device__ __forceinline__ void tsit5_stages(Tsit5Lane<S, K, N>& L, double t, double dt, double (&ea)[N]) {
     if constexpr (sizeof(K) < sizeof(S)) {
-        tsit5_perform_step_mixed(L, P);
+        tsit5_stages_mixed(L, t, dt, ea);
         return;
     }
     typedef Tsit5Tab T;
-    const double t = L.c.t, dt = L.c.dt;
-    K tmp[N];
-    double ea[N];  // embedded error sum bt1*k1 + ... + bt7*k7, accumulated in FP64 as stages appear
+    K tmp[N];   // the error sum is accumulated in FP64 as stages appear
     const K a = (K)(dt * T::a21);
 #pragma unroll
     for (int i = 0; i < N; i++) {
@@ -1038,10 +1070,17 @@ __device__ __forceinline__ void tsit5_perform_step(Tsit5Lane<S, K, N>& L, const 
 #pragma unroll
     for (int i = 0; i < N; i++) tmp[i] = (K)L.u[i];
     odemi_f<K>(L.k7, tmp, L.p, (K)(t + dt));
-    L.c.nf += 6;
 #pragma unroll
     for (int i = 0; i < N; i++) ea[i] = dt * fma(T::bt7, (double)L.k7[i], ea[i]);
-    L.c.EEst = residual_norm<N>(ea, L.uprev, L.u, P.abstol, P.reltol);
+}
+
+template <typename S, typename K, int N>
+__device__ __forceinline__ void tsit5_perform_step(Tsit5Lane<S, K, N>& L, const Params& P) {
+    double ea[N];
+    tsit5_stages(L, L.c.t, L.c.dt, ea);
+    L.c.nf += 6;
+    if constexpr (sizeof(K) < sizeof(S)) L.c.EEst = residual_norm_nr<N>(ea, L.uprev, L.u, P.abstol, P.reltol);
+    else L.c.EEst = residual_norm<N>(ea, L.uprev, L.u, P.abstol, P.reltol);
 }
 
 // interpolants.jl:52-64 (@evalpoly Horner via muladd), FP64 evaluation.
@@ -1496,9 +1535,6 @@ __device__ __forceinline__ int tsit5_attempt(Tsit5Lane<S, K, N>& L, const Params
 #endif
             c.dt = c.dtpropose;
             apply_step_tstop_clip(c);
-        } else {
-            if (c.isout) c.dt = c.dt * kc.qmin;   // handle_step_rejection! (integrator_utils.jl:135-136)
-            else reject_controller<(sizeof(K) < sizeof(S))>(c, kc);
         }
     }
     c.iter++;
@@ -1539,8 +1575,196 @@ __device__ __forceinline__ int tsit5_attempt(Tsit5Lane<S, K, N>& L, const Params
         if (term) return RC_TERMINATED;
     } else {
         c.nreject++;
+        reject_controller<HW>(c, kc);
     }
     return (c.tdir * c.t < c.tdir * c.tf) ? 0 : RC_SUCCESS;
+}
+
+// ---------------------------------------------------------------------------
+// The common attempt, without the rules that cannot bite.
+//
+// Through the complete rules an attempt issues ~590 vector and ~240 scalar
+// instructions on Lorenz, ~150 of them stage arithmetic: Julia's NaN-aware min
+// and max and eps as selects, three tests of dt against eps and dtmin, IEEE
+// divisions and square root with scaling and fix-up, a finiteness test, and a
+// branch with its mask bookkeeping around each.  A wave alone on its SIMD issues
+// one instruction per ~6 cycles whatever their dependences, and four waves share
+// the SIMD's one vector issue per 4 cycles, so small and large batches alike pay
+// by the count.
+//
+// tsit5_attempt_fast makes the same attempt, bit for bit, under conditions that
+// it checks: the trajectory is regular (FastCtl::bound, set once), dt stays
+// above `bound` -- then dt > eps(t) and dt > dtmin need no test, max(eps(t),
+// dtmin) never acts and no quotient leaves div_nr's range -- and the error sum
+// is finite and below 2^1000, which also proves u and all stages finite.  A lane
+// whose attempt fails a check makes it again by the complete rules
+// (tsit5_attempt), from the state that the checks left alone.
+//
+// State between attempts: t, uprev (the current solution), k1 = f(uprev),
+// erroldp and FastCtl; the other counters follow from `att` and c.nreject.
+// ---------------------------------------------------------------------------
+struct FastCtl {
+    double x;       // next |dt|, < 0 after a rejected attempt
+    double tol;     // 100 eps(max(|t|, |tf|)), constant while |t| <= |tf|
+    double bound;   // a dt above it is beyond the reach of eps(t) and dtmin; inf: irregular trajectory
+    double snext;   // next save time; inf: none, -inf: every step (saving kernels)
+    int att;        // attempts made
+};
+// a / b for a constant b, rb = 1.0 / b folded by the compiler
+__device__ __forceinline__ double div_const(double a, double b, double rb) { return div_by_rcp(a, b, rb); }
+
+__device__ __forceinline__ void fast_next_save(FastCtl& F, const Ctl& c, const Params& P) {
+    F.snext = P.save_everystep ? -__builtin_huge_val()
+                               : (c.spos != c.send) ? P.saveat[c.spos] : __builtin_huge_val();
+}
+// FastCtl from a controller state between attempts (counters whole) ...
+__device__ __forceinline__ void fast_from_ctl(FastCtl& F, const Ctl& c) {
+    F.att = c.naccept + c.nreject;
+    F.x = (F.att == 0) ? c.tdir * c.dt : c.accept_step ? fabs(c.dtpropose) : -fabs(c.dt);
+}
+// ... and back.  dtpropose's lower bound (accept_controller) acts here.
+__device__ __forceinline__ void fast_to_ctl(const FastCtl& F, Ctl& c, const Params& P) {
+    c.iter = F.att;
+    c.naccept = F.att - c.nreject;
+    c.accept_step = (F.att > 0 && F.x > 0.0) ? 1 : 0;
+    c.success_iter = c.naccept - c.accept_step;
+    c.dt = c.tdir * ((F.att == 0) ? F.x : fabs(F.x));
+    c.dtpropose = c.accept_step ? c.tdir * jl_max(F.x, fabs(jl_max(jl_eps(c.t), P.dtmin))) : c.dt;
+}
+// Once per trajectory (or serving tick), from a whole controller state.
+// Regular: forward, times of ordinary size with |t| <= |tf|, tolerances that
+// keep the error norm's denominators in range, no user stopping times.
+template <bool SAVES>
+__device__ __forceinline__ void fast_init(FastCtl& F, const Ctl& c, const Params& P) {
+    fast_from_ctl(F, c);
+    const double atf = fabs(c.tf);
+    const bool regular = P.ntstops == 0 && P.abstol >= 0x1p-500 && P.abstol <= 0x1p+500 && P.reltol >= 0.0 &&
+                         P.reltol <= 0.25 && fabs(P.dtmin) <= 0x1p+500 && c.tdir > 0.0 && atf >= 0x1p-500 &&
+                         atf <= 0x1p+500 && fabs(c.t) <= atf && c.dtmax <= 0x1p+600 && fabs(c.dt) <= 0x1p+600;
+    const double e = jl_eps(atf);
+    F.tol = 100.0 * e;
+    F.bound = regular ? fmax(e, fabs(P.dtmin)) : __builtin_huge_val();
+    if (regular && F.att == 0) F.x = fmin(F.x, c.dtmax);   // the first loop header's min(dtmax, dt)
+    if (SAVES) fast_next_save(F, c, P);
+}
+
+// The controller's part of a fast attempt: the PI quotient and the step's fate
+// from EEst.  Returns the divisor of dt for the next attempt, negative for a
+// rejection; `first`: no attempt was accepted before this one.
+template <bool HW>
+__device__ __forceinline__ double fast_controller(double EEst, float erroldp, bool first, const CtlConst& k, float& lg) {
+    lg = fast_log2<HW>(EEst);   // EEst = 0 ends at the lower limit of q, as by the complete rules
+    const double q11 = pow_of_log2<HW>(k.beta1, lg);
+    double x;
+    if constexpr (HW) x = div_nr(q11, (double)erroldp * k.gamma);
+    else x = div_const(div_f32_values(q11, erroldp), k.gamma, 1.0 / k.gamma);
+    const double lo = first ? 1.0 / k.qmax_first : 1.0 / k.qmax;
+    double q = fmin(fmax(x, lo), 1.0 / k.qmin);
+    if (k.qsteady_max > 1.0) q = (q >= k.qsteady_min && q <= k.qsteady_max) ? 1.0 : q;
+    const double rej = fmin(1.0 / k.qmin, div_const(q11, k.gamma, 1.0 / k.gamma));
+    return (EEst <= 1.0) ? q : -rej;
+}
+// EEst = sqrt(s / N) of the error sum s, 0 <= s < 2^1000.  Below 2^-700 any root
+// below the smallest Float32 serves: the controller takes EEst to Float32.
+template <bool HW, int N>
+__device__ __forceinline__ double fast_eest(double s) {
+    const double m = HW ? s * (1.0 / (double)(N > 1 ? N : 1))
+                        : (N > 1) ? div_const(s, (double)N, 1.0 / (double)N) : s;
+    return sqrt_inrange(fmax(m, 0x1p-700));
+}
+// sum of (e / (abstol + reltol max(|u0|, |u1|)))^2, NaN when any u1 is not finite
+template <int N>
+__device__ __forceinline__ double fast_error_sum(const double (&e)[N], const double (&u0)[N], const double (&u1)[N],
+                                                 double abstol, double reltol) {
+    double s = 0.0;
+#pragma unroll
+    for (int i = 0; i < N; i++) s = fma(u1[i], 0.0, s);
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        const double r = div_nr(e[i], fma(fmax(fabs(u0[i]), fabs(u1[i])), reltol, abstol));
+        s = fma(r, r, s);
+    }
+    return s;
+}
+
+// One attempt.  0: running, RC_SUCCESS: the end was reached, -1: a check failed
+// and the attempt is still to be made (tsit5_attempt_full).
+template <bool SAVES, typename K, int N>
+__device__ __forceinline__ int tsit5_attempt_fast(Tsit5Lane<double, K, N>& L, FastCtl& F, const Params& P, i64 j,
+                                                  int itmax) {
+    constexpr bool HW = sizeof(K) < sizeof(double);
+    const CtlConst kc = ctl_const(false);
+    Ctl& c = L.c;
+    const double left = c.tf - c.t;
+    const double dt = fmin(fabs(F.x), left);
+    // L.u keeps a rejected attempt's state until the next step is sure to be made
+    if (!((dt > F.bound) & (F.att < itmax))) return -1;
+    const bool last = !(dt + F.tol < left);
+    double ea[N];
+    tsit5_stages(L, c.t, dt, ea);
+    const double s = fast_error_sum<N>(ea, L.uprev, L.u, P.abstol, P.reltol);
+    const double EEst = fast_eest<HW, N>(s);
+    float lg;
+    const double d = fast_controller<HW>(EEst, c.erroldp, F.att == c.nreject, kc, lg);
+    const double dtn = div_nr(dt, d);
+    if (!(s < 0x1p+1000)) return -1;
+    F.att++;
+    if (!(d > 0.0)) {
+        c.nreject++;
+        F.x = dtn;
+        return 0;
+    }
+    const double tn = last ? c.tf : c.t + dt;
+    if (SAVES) {
+        if (tn >= F.snext) {
+            c.tprev = c.t;
+            c.dt = (last && F.att == 1) ? F.x : dt;   // a flagged step restores the unclipped dt
+            c.t = tn;
+            tsit5_savevalues(L, P, j);
+            fast_next_save(F, c, P);
+        }
+    }
+    c.t = tn;
+#pragma unroll
+    for (int i = 0; i < N; i++) { L.uprev[i] = L.u[i]; L.k1[i] = L.k7[i]; }
+    c.erroldp = (EEst > kc.qoldinit) ? pow_of_log2<HW>(kc.beta2, lg) : erroldp_init<HW>();
+    F.x = fmin(dtn, c.dtmax);
+    return last ? RC_SUCCESS : 0;
+}
+// The same attempt by the complete rules.
+template <bool SAVES, typename K, int N>
+__device__ __forceinline__ int tsit5_attempt_full(Tsit5Lane<double, K, N>& L, FastCtl& F, const Params& P, i64 j) {
+    Ctl& c = L.c;
+    const int att0 = F.att;
+    fast_to_ctl(F, c, P);
+    if (c.accept_step) {
+#pragma unroll
+        for (int i = 0; i < N; i++) { L.u[i] = L.uprev[i]; L.k7[i] = L.k1[i]; }
+    }
+    const int rc = tsit5_attempt<SAVES>(L, P, j);
+    fast_from_ctl(F, c);
+    c.nf -= 6 * (F.att - att0);
+    if (c.accept_step) {
+#pragma unroll
+        for (int i = 0; i < N; i++) { L.uprev[i] = L.u[i]; L.k1[i] = L.k7[i]; }
+    }
+    if (SAVES) fast_next_save(F, c, P);
+    return rc;
+}
+// The counters that FastCtl::att stands for (c.nf holds the rest meanwhile).
+__device__ __forceinline__ void fast_counts(const FastCtl& F, Ctl& c) {
+    c.naccept = F.att - c.nreject;
+    c.nf += 6 * F.att;
+}
+// Modules whose attempts run user hooks (callbacks, isoutofdomain) keep to the
+// complete rules.
+#if defined(ODEMI_NDCB) || defined(ODEMI_NCCB) || defined(ODEMI_HAS_ISOUT)
+constexpr bool kFastAttempts = false;
+#else
+constexpr bool kFastAttempts = true;
+#endif
+__device__ __forceinline__ int fast_itmax(const Params& P) {
+    return (int)(P.maxiters < 0x7fffffffLL ? P.maxiters : 0x7fffffffLL);
 }
 
 // ---------------------------------------------------------------------------
@@ -1601,6 +1825,9 @@ __device__ void tsit5_persistent(const Params& P) {
     WaveQueue q;
     bool active = false, exhausted = false;
     i64 j = 0, js = 0;
+    FastCtl F;
+    const int itmax = fast_itmax(P);
+    (void)F; (void)itmax;
     for (;;) {
         bool need = refill_now(!active && !exhausted, active);
         i64 slot = wave_fetch(&P.counters[0], q, need);
@@ -1609,6 +1836,10 @@ __device__ void tsit5_persistent(const Params& P) {
                 js = slot;
                 j = P.order ? P.order[slot] : slot;
                 tsit5_init(L, P, j, slot);
+                if constexpr (kFastAttempts) {
+                    fast_init<SAVES>(F, L.c, P);
+                    L.c.nf -= 6 * F.att;
+                }
                 active = true;
             } else {
                 exhausted = true;
@@ -1616,8 +1847,17 @@ __device__ void tsit5_persistent(const Params& P) {
         }
         if (__ballot(active) == 0) break;
         if (active) {
-            int rc = tsit5_attempt<SAVES>(L, P, j);
+            int rc;
+            if constexpr (kFastAttempts) {
+                // until a lane of the wave ends
+                do rc = tsit5_attempt_fast<SAVES>(L, F, P, j, itmax);
+                while (__ballot(rc != 0) == 0);
+                if (__builtin_expect(rc < 0, 0)) rc = tsit5_attempt_full<SAVES>(L, F, P, j);
+            } else {
+                rc = tsit5_attempt<SAVES>(L, P, j);
+            }
             if (rc) {
+                if constexpr (kFastAttempts) fast_counts(F, L.c);
                 if (!SAVES && P.rec_out) finish_lane_rec<N>(L.c, P, js, L.u, rc);
                 else finish_lane<N>(L.c, P, j, L.u, rc);
                 active = false;
@@ -1627,7 +1867,7 @@ __device__ void tsit5_persistent(const Params& P) {
 }
 
 // Plain engine: one kernel launch per step attempt, state in HBM.
-// st_scalar rows: t dt dtpropose tprev last_event_error tf dtmax EEst q11 errold
+// st_scalar rows: t dt dtpropose tprev last_event_error tf dtmax EEst - fastpower(errold, beta2)
 // st_int rows: iter success_iter accept_step next_step_tstop nf naccept nreject done
 //               saveat cursor, njacs nw nsolve (Rodas5P), tstops cursor,
 //               isout | reeval_fsal << 1, ncondition, event_last | sim_mask << 8
@@ -1640,7 +1880,7 @@ __device__ __forceinline__ void plain_load_ctl(Ctl& c, const Params& P, i64 j) {
     c.last_event_error = s[4 * M + j];
     c.tf = s[5 * M + j]; c.dtmax = s[6 * M + j];
     c.tdir = (c.tf < P.t0[j]) ? -1.0 : 1.0;
-    c.EEst = s[7 * M + j]; c.q11 = s[8 * M + j]; c.errold = s[9 * M + j];
+    c.EEst = s[7 * M + j]; c.q11 = 1.0; c.erroldp = (float)s[9 * M + j];
     const int* q = P.st_int;
     c.iter = q[0 * M + j]; c.success_iter = q[1 * M + j]; c.accept_step = q[2 * M + j];
     c.next_step_tstop = q[3 * M + j]; c.nf = q[4 * M + j]; c.naccept = q[5 * M + j];
@@ -1663,7 +1903,7 @@ __device__ __forceinline__ void plain_load_ctl(Ctl& c, const Params& P, i64 j) {
     c.event_last = q[15 * M + j] & 0xff;
     c.sim_mask = (unsigned)q[15 * M + j] >> 8;
     c.njacs = 0; c.nw = 0; c.nsolve = 0;
-    c.erroldp = __builtin_nanf(""); c.lgEEst = 0.0f;
+    c.lgEEst = 0.0f;
 }
 template <int N>
 __device__ __forceinline__ void plain_store_ctl(const Ctl& c, const Params& P, i64 j, int done) {
@@ -1672,7 +1912,7 @@ __device__ __forceinline__ void plain_store_ctl(const Ctl& c, const Params& P, i
     s[0 * M + j] = c.t; s[1 * M + j] = c.dt; s[2 * M + j] = c.dtpropose; s[3 * M + j] = c.tprev;
     s[4 * M + j] = c.last_event_error;
     s[5 * M + j] = c.tf; s[6 * M + j] = c.dtmax;
-    s[7 * M + j] = c.EEst; s[8 * M + j] = c.q11; s[9 * M + j] = c.errold;
+    s[7 * M + j] = c.EEst; s[9 * M + j] = (double)c.erroldp;
     int* q = P.st_int;
     q[0 * M + j] = c.iter; q[1 * M + j] = c.success_iter; q[2 * M + j] = c.accept_step;
     q[3 * M + j] = c.next_step_tstop; q[4 * M + j] = c.nf; q[5 * M + j] = c.naccept;
@@ -1823,7 +2063,7 @@ struct RodasLane {
 
 template <typename F, int N>
 __device__ __forceinline__ void rodas_init(RodasLane<F, N>& L, const Params& P, i64 j) {
-    ctl_init(L.c, P, j);
+    ctl_init(L.c, P, j, sizeof(F) < sizeof(double));
 #pragma unroll
     for (int i = 0; i < N; i++) { L.u[i] = P.u0[(i64)i * P.N + j]; L.uprev[i] = L.u[i]; L.dT[i] = 0.0; }
 #pragma unroll
@@ -2119,9 +2359,6 @@ __device__ __forceinline__ int rodas_attempt(RodasLane<F, N>& L, const Params& P
             for (int i = 0; i < N; i++) L.uprev[i] = L.u[i];
             c.dt = c.dtpropose;
             apply_step_tstop_clip(c);
-        } else {
-            if (c.isout) c.dt = c.dt * kc.qmin;   // handle_step_rejection! (integrator_utils.jl:135-136)
-            else reject_controller<(sizeof(F) < sizeof(double))>(c, kc);
         }
     }
     c.iter++;
@@ -2162,6 +2399,7 @@ __device__ __forceinline__ int rodas_attempt(RodasLane<F, N>& L, const Params& P
         if (term) return RC_TERMINATED;
     } else {
         c.nreject++;
+        reject_controller<HW>(c, kc);
     }
     return (c.tdir * c.t < c.tdir * c.tf) ? 0 : RC_SUCCESS;
 }
@@ -2323,14 +2561,38 @@ __device__ void tsit5_serve_tick(const Params& P0) {
     }
 #pragma unroll
     for (int k = 0; k < ODEMI_NP; k++) L.p[k] = (K)((k < P.np) ? P.p[(i64)k * P.N + j] : 0.0);
+    FastCtl F;
+    const int itmax = fast_itmax(P);
+    (void)F; (void)itmax;
+    if constexpr (kFastAttempts) {
+        if (L.c.accept_step) {   // to the state between fast attempts
+#pragma unroll
+            for (int i = 0; i < N; i++) { L.uprev[i] = L.u[i]; L.k1[i] = L.k7[i]; }
+        }
+        fast_init<SAVES>(F, L.c, P);
+        L.c.nf -= 6 * F.att;
+    }
     for (int a = 0; a < P.tick_attempts; a++) {
-        int rc = tsit5_attempt<SAVES>(L, P, j);
+        int rc;
+        if constexpr (kFastAttempts) {
+            rc = tsit5_attempt_fast<SAVES>(L, F, P, j, itmax);
+            if (__builtin_expect(rc < 0, 0)) rc = tsit5_attempt_full<SAVES>(L, F, P, j);
+        } else {
+            rc = tsit5_attempt<SAVES>(L, P, j);
+        }
         if (rc) {
+            if constexpr (kFastAttempts) fast_counts(F, L.c);
             finish_lane<N>(L.c, P, j, L.u, rc);
             plain_store_ctl<N>(L.c, P, j, 0);
             atomicAdd(&P.req_done[P.slot_req[j]], 1ULL);
             return;
         }
+    }
+    if constexpr (kFastAttempts) {
+        fast_to_ctl(F, L.c, P);
+        fast_counts(F, L.c);
+#pragma unroll
+        for (int i = 0; i < N; i++) { L.u[i] = L.uprev[i]; L.k7[i] = L.k1[i]; }
     }
     plain_store_ctl<N>(L.c, P, j, 1);
     tsit5_store_state(L, P, j);

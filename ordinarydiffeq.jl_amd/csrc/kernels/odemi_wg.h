@@ -949,12 +949,6 @@ __device__ __forceinline__ int wg_run(const WGPtrs& S, const Params& P, i64 j, i
                 for (int i = tid; i < n; i += NT) uprev[i] = u[i];
                 c.dt = c.dtpropose;
                 apply_step_tstop_clip(c);
-            } else {
-#ifdef ODEMI_HAS_ISOUT_WG
-                if (c.isout) c.dt = c.dt * kc.qmin;   // handle_step_rejection! (integrator_utils.jl:135-136)
-                else
-#endif
-                reject_controller(c, kc);
             }
         }
         c.iter++;
@@ -1151,6 +1145,7 @@ __device__ __forceinline__ int wg_run(const WGPtrs& S, const Params& P, i64 j, i
 #endif
         } else {
             c.nreject++;
+            reject_controller(c, kc);
         }
     }
     return rc;
