@@ -331,36 +331,26 @@ __constant__ double kTsitR[7][4] = {
 struct RodasTab {
     static constexpr double gamma = 0.21193756319429014;
 };
-__constant__ double kRA[8][8] = {
-    {0, 0, 0, 0, 0, 0, 0, 0},
-    {3.0, 0, 0, 0, 0, 0, 0, 0},
-    {2.849394379747939, 0.45842242204463923, 0, 0, 0, 0, 0, 0},
-    {-6.954028509809101, 2.489845061869568, -10.358996098473584, 0, 0, 0, 0, 0},
-    {2.8029986275628964, 0.5072464736228206, -0.3988312541770524, -0.04721187230404641, 0, 0, 0, 0},
-    {-7.502846399306121, 2.561846144803919, -11.627539656261098, -0.18268767659942256,
-     0.030198172008377946, 0, 0, 0},
-    {-7.502846399306121, 2.561846144803919, -11.627539656261098, -0.18268767659942256,
-     0.030198172008377946, 1, 0, 0},
-    {-7.502846399306121, 2.561846144803919, -11.627539656261098, -0.18268767659942256,
-     0.030198172008377946, 1, 1, 0},
+// One 128-byte row a stage: a[s][0..6], C[s][0..6], c[s], d[s] (two scalar loads
+// where a kernel reads a row at its stage).
+__constant__ double kRStage[8][16] = {
+    {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0.21193756319429014},
+    {3.0, 0, 0, 0, 0, 0, 0, -14.155112264123755, 0, 0, 0, 0, 0, 0, 0.6358126895828704, -0.42387512638858027},
+    {2.849394379747939, 0.45842242204463923, 0, 0, 0, 0, 0, -17.97296035885952, -2.859693295451294, 0, 0, 0, 0, 0,
+     0.4095798393397535, -0.3384627126235924},
+    {-6.954028509809101, 2.489845061869568, -10.358996098473584, 0, 0, 0, 0, 147.12150275711716, -1.41221402718213,
+     71.68940251302358, 0, 0, 0, 0, 0.9769306725060716, 1.8046452872882734},
+    {2.8029986275628964, 0.5072464736228206, -0.3988312541770524, -0.04721187230404641, 0, 0, 0, 165.43517024871676,
+     -0.4592823456491126, 42.90938336958603, -5.961986721573306, 0, 0, 0, 0.4288403609558664, 2.325825639765069},
+    {-7.502846399306121, 2.561846144803919, -11.627539656261098, -0.18268767659942256, 0.030198172008377946, 0, 0,
+     24.854864614690072, -3.0009227002832186, 47.4931110020768, 5.5814197821558125, -0.6610691825249471, 0, 0, 1, 0},
+    {-7.502846399306121, 2.561846144803919, -11.627539656261098, -0.18268767659942256, 0.030198172008377946, 1, 0,
+     30.91273214028599, -3.1208243349937974, 77.79954646070892, 34.28646028294783, -19.097331116725623,
+     -28.087943162872662, 0, 1, 0},
+    {-7.502846399306121, 2.561846144803919, -11.627539656261098, -0.18268767659942256, 0.030198172008377946, 1, 1,
+     37.80277123390563, -3.2571969029072276, 112.26918849496327, 66.9347231244047, -40.06618937091002,
+     -54.66780262877968, -9.48861652309627, 1, 0},
 };
-__constant__ double kRC[8][7] = {
-    {0, 0, 0, 0, 0, 0, 0},
-    {-14.155112264123755, 0, 0, 0, 0, 0, 0},
-    {-17.97296035885952, -2.859693295451294, 0, 0, 0, 0, 0},
-    {147.12150275711716, -1.41221402718213, 71.68940251302358, 0, 0, 0, 0},
-    {165.43517024871676, -0.4592823456491126, 42.90938336958603, -5.961986721573306, 0, 0, 0},
-    {24.854864614690072, -3.0009227002832186, 47.4931110020768, 5.5814197821558125,
-     -0.6610691825249471, 0, 0},
-    {30.91273214028599, -3.1208243349937974, 77.79954646070892, 34.28646028294783,
-     -19.097331116725623, -28.087943162872662, 0},
-    {37.80277123390563, -3.2571969029072276, 112.26918849496327, 66.9347231244047,
-     -40.06618937091002, -54.66780262877968, -9.48861652309627},
-};
-__constant__ double kRc[8] = {0, 0.6358126895828704, 0.4095798393397535, 0.9769306725060716,
-                              0.4288403609558664, 1, 1, 1};
-__constant__ double kRd[8] = {0.21193756319429014, -0.42387512638858027, -0.3384627126235924,
-                              1.8046452872882734, 2.325825639765069, 0, 0, 0};
 __constant__ double kRH[3][8] = {
     {25.948786856663858, -2.5579724845846235, 10.433815404888879, -2.3679251022685204,
      0.524948541321073, 1.1241088310450404, 0.4272876194431874, -0.17202221070155493},
@@ -2161,7 +2151,7 @@ __device__ __forceinline__ void rodas_perform_step(RodasLane<F, N>& L, const Par
         odemi_tgrad<double>(L.dT, L.uprev, L.p, t);
         if (!ODEMI_HAS_TGRAD) c.nf += 1;
     }
-    const double dtd0 = dt * kRd[0];
+    const double dtd0 = dt * kRStage[0][15];
 #pragma unroll
     for (int i = 0; i < N; i++) lt[i] = fsal[i] + dtd0 * L.dT[i];
 #pragma unroll
@@ -2179,17 +2169,17 @@ __device__ __forceinline__ void rodas_perform_step(RodasLane<F, N>& L, const Par
         for (int i = 0; i < N; i++) {
             double acc = L.uprev[i];
 #pragma unroll
-            for (int q = 0; q < s; q++) acc = fma(kRA[s][q], L.ks[q][i], acc);
+            for (int q = 0; q < s; q++) acc = fma(kRStage[s][q], L.ks[q][i], acc);
             L.u[i] = acc;
         }
-        odemi_f<double>(du, L.u, L.p, fma(kRc[s], dt, t));
+        odemi_f<double>(du, L.u, L.p, fma(kRStage[s][14], dt, t));
         c.nf += 1;
-        const double dtds = dt * kRd[s];
+        const double dtds = dt * kRStage[s][15];
 #pragma unroll
         for (int i = 0; i < N; i++) {
             double acc = fma(dtds, L.dT[i], du[i]);
 #pragma unroll
-            for (int q = 0; q < s; q++) acc = fma(kRC[s][q] * idt, L.ks[q][i], acc);
+            for (int q = 0; q < s; q++) acc = fma(kRStage[s][7 + q] * idt, L.ks[q][i], acc);
             lt[i] = acc;
         }
         rodas_wsolve<F, N>(W, LU, piv, lt, P.refine_sweeps);
@@ -2201,7 +2191,7 @@ __device__ __forceinline__ void rodas_perform_step(RodasLane<F, N>& L, const Par
     for (int i = 0; i < N; i++) {
         double acc = L.uprev[i];
 #pragma unroll
-        for (int q = 0; q < 7; q++) acc = fma(kRA[7][q], L.ks[q][i], acc);
+        for (int q = 0; q < 7; q++) acc = fma(kRStage[7][q], L.ks[q][i], acc);
         acc = fma(1.0, L.ks[7][i], acc);
         L.u[i] = acc;
     }
@@ -2311,16 +2301,16 @@ __device__ void rodas_addsteps(RodasLane<F, N>& L, const Params& P) {
         for (int i = 0; i < N; i++) {
             double acc = L.uprev[i];
 #pragma unroll
-            for (int q = 0; q < s; q++) acc = acc + kRA[s][q] * L.ks[q][i];
+            for (int q = 0; q < s; q++) acc = acc + kRStage[s][q] * L.ks[q][i];
             st[i] = acc;
         }
-        odemi_f<double>(du, st, L.p, t + kRc[s] * dt);
-        const double dtds = dt * kRd[s];
+        odemi_f<double>(du, st, L.p, t + kRStage[s][14] * dt);
+        const double dtds = dt * kRStage[s][15];
 #pragma unroll
         for (int i = 0; i < N; i++) {
             double acc = du[i] + dtds * L.dT[i];
 #pragma unroll
-            for (int q = 0; q < s; q++) acc = acc + (kRC[s][q] / dt) * L.ks[q][i];
+            for (int q = 0; q < s; q++) acc = acc + (kRStage[s][7 + q] / dt) * L.ks[q][i];
             lt[i] = acc;
         }
         rodas_wsolve<F, N>(W, LU, piv, lt, P.refine_sweeps);
@@ -2404,12 +2394,323 @@ __device__ __forceinline__ int rodas_attempt(RodasLane<F, N>& L, const Params& P
     return (c.tdir * c.t < c.tdir * c.tf) ? 0 : RC_SUCCESS;
 }
 
+// ---------------------------------------------------------------------------
+// The common Rodas5P attempt (see tsit5_attempt_fast for the conditions and the
+// hand-over to the complete rules).  What the complete form spends beside the
+// arithmetic: 24 IEEE divisions of the eight substitutions by the same N pivots
+// (here one refined reciprocal a pivot and 3 instructions a quotient), row
+// exchanges as selects in every substitution (here skipped while no lane of the
+// wave exchanged rows), the tableau held in spilled scalar registers (196
+// v_readlane an attempt; here two scalar loads a stage, kept from being hoisted),
+// stage sums of the last stages that share their first five terms, and the
+// controller's rules.
+// ---------------------------------------------------------------------------
+typedef const __attribute__((address_space(4))) double* const_f64_ptr;
+
+// Dense LU on registers: the arithmetic of lu_factor_reg / lu_solve_reg.
+template <typename T, int N>
+struct FastLu {
+    T A[N][N];
+    T r[N];        // reciprocals of the pivots (T float: the hardware estimate, as lu_solve_reg uses it)
+    int piv[N];
+    bool swaps;    // a lane of the wave exchanged rows (wave-uniform)
+};
+template <typename T, int N>
+__device__ __forceinline__ void fast_lu_factor(FastLu<T, N>& L) {
+    bool moved = false;
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+        int p = k;
+        T amax = fabs(L.A[k][k]);
+#pragma unroll
+        for (int i = k + 1; i < N; i++) {
+            const T v = fabs(L.A[i][k]);
+            if (v > amax) { amax = v; p = i; }
+        }
+        L.piv[k] = p;
+        if (k + 1 < N && __ballot(p != k) != 0) {
+            moved = true;
+#pragma unroll
+            for (int i = k + 1; i < N; i++) {
+                const bool s = (p == i);
+#pragma unroll
+                for (int c = 0; c < N; c++) {
+                    const T a = L.A[k][c], b = L.A[i][c];
+                    L.A[k][c] = s ? b : a;
+                    L.A[i][c] = s ? a : b;
+                }
+            }
+        }
+        T inv;
+        if constexpr (sizeof(T) == sizeof(float)) {
+            L.r[k] = __builtin_amdgcn_rcpf(L.A[k][k]);
+            inv = L.r[k];
+        } else {
+            L.r[k] = rcp_nr(L.A[k][k]);
+            inv = fma(fma(-L.A[k][k], L.r[k], 1.0), L.r[k], L.r[k]);   // div_nr(1, pivot)
+        }
+#pragma unroll
+        for (int i = k + 1; i < N; i++) {
+            const T l = L.A[i][k] * inv;
+            L.A[i][k] = l;
+#pragma unroll
+            for (int c = k + 1; c < N; c++) L.A[i][c] = fma(-l, L.A[k][c], L.A[i][c]);
+        }
+    }
+    L.swaps = moved;
+}
+// emin: least binary exponent among the dividends (a zero has none)
+template <typename T, int N>
+__device__ __forceinline__ void fast_lu_solve(const FastLu<T, N>& L, T (&b)[N], int& emin) {
+    if (L.swaps) {
+#pragma unroll
+        for (int k = 0; k < N; k++) {
+#pragma unroll
+            for (int i = k + 1; i < N; i++) {
+                const bool s = (L.piv[k] == i);
+                const T x = b[k], y = b[i];
+                b[k] = s ? y : x;
+                b[i] = s ? x : y;
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 1; i < N; i++) {
+        T acc = b[i];
+#pragma unroll
+        for (int c = 0; c < i; c++) acc = fma(-L.A[i][c], b[c], acc);
+        b[i] = acc;
+    }
+#pragma unroll
+    for (int c = N - 1; c >= 0; c--) {
+        if constexpr (sizeof(T) == sizeof(float)) {
+            b[c] = b[c] * L.r[c];
+        } else {
+            emin = min(emin, __builtin_amdgcn_frexp_exp(b[c]));
+            b[c] = div_by_rcp(b[c], L.A[c][c], L.r[c]);
+        }
+#pragma unroll
+        for (int i = 0; i < c; i++) b[i] = fma(-L.A[i][c], b[c], b[i]);
+    }
+}
+template <typename F, int N>
+__device__ __forceinline__ void fast_wsolve(const double (&W)[N][N], const FastLu<F, N>& LU, double (&b)[N], int sweeps,
+                                            int& emin) {
+    if constexpr (sizeof(F) == sizeof(double)) {
+        fast_lu_solve<double, N>(LU, b, emin);
+    } else {
+        F xf[N];
+        double x[N];
+#pragma unroll
+        for (int i = 0; i < N; i++) xf[i] = (F)b[i];
+        fast_lu_solve<F, N>(LU, xf, emin);
+#pragma unroll
+        for (int i = 0; i < N; i++) x[i] = (double)xf[i];
+        for (int s = 0; s < sweeps; s++) {
+#pragma unroll
+            for (int i = 0; i < N; i++) {
+                double acc = b[i];
+#pragma unroll
+                for (int c = 0; c < N; c++) acc = fma(-W[i][c], x[c], acc);
+                xf[i] = (F)acc;
+            }
+            fast_lu_solve<F, N>(LU, xf, emin);
+#pragma unroll
+            for (int i = 0; i < N; i++) x[i] = x[i] + (double)xf[i];
+        }
+#pragma unroll
+        for (int i = 0; i < N; i++) b[i] = x[i];
+    }
+}
+
+// fma(h, dT, x), or x where the traced time derivative is zero throughout
+__device__ __forceinline__ double add_tgrad(double h, double dT, double x) {
+    if (__builtin_constant_p(dT) && dT == 0.0) return x;
+    return fma(h, dT, x);
+}
+
+template <typename F, int N>
+__device__ __forceinline__ int rodas_attempt_fast(RodasLane<F, N>& L, FastCtl& FC, const Params& P, i64 j, int itmax) {
+    constexpr bool HW = sizeof(F) < sizeof(double);
+    const CtlConst kc = ctl_const(true);
+    Ctl& c = L.c;
+    const double left = c.tf - c.t;
+    const double dt = fmin(fabs(FC.x), left);
+    if (!((dt > FC.bound) & (dt < 0x1p+450) & (dt > 0x1p-450) & (FC.att < itmax))) return -1;
+    const bool last = !(dt + FC.tol < left);
+    const double t = c.t;
+    // 1/dt and 1/(dt gamma): rcp_nr for the mixed engine, the IEEE quotient for FP64
+    const double dtgamma = dt * RodasTab::gamma;
+    double idt = rcp_nr(dt), sigma = rcp_nr(dtgamma);
+    if constexpr (!HW) {
+        idt = fma(fma(-dt, idt, 1.0), idt, idt);
+        sigma = fma(fma(-dtgamma, sigma, 1.0), sigma, sigma);
+    }
+    // the tableau's address, opaque once an attempt, so that its rows are loaded
+    // where they are used
+    const_f64_ptr rows = (const_f64_ptr)&kRStage[0][0];
+    asm volatile("" : "+s"(rows));
+    double fsal[N], du[N], x[N], dT[N], J[N][N], W[N][N], ks[8][N];
+    FastLu<F, N> LU;
+    odemi_f<double>(fsal, L.uprev, L.p, t);
+#pragma unroll
+    for (int a = 0; a < N; a++)
+#pragma unroll
+        for (int b = 0; b < N; b++) J[a][b] = 0.0;
+    odemi_jac<double>(&J[0][0], L.uprev, L.p, t);
+#pragma unroll
+    for (int i = 0; i < N; i++) dT[i] = 0.0;
+    odemi_tgrad<double>(dT, L.uprev, L.p, t);
+#pragma unroll
+    for (int a = 0; a < N; a++)
+#pragma unroll
+        for (int b = 0; b < N; b++) {
+            W[a][b] = (a == b) ? J[a][b] - sigma : J[a][b];   // fma(-1, sigma, J)
+            LU.A[a][b] = (F)W[a][b];
+        }
+    fast_lu_factor<F, N>(LU);
+    int emin = 0;
+    const double dtd0 = dt * rows[15];
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        const bool zero = __builtin_constant_p(dT[i]) && dT[i] == 0.0;
+        x[i] = zero ? fsal[i] : fsal[i] + dtd0 * dT[i];
+    }
+    fast_wsolve<F, N>(W, LU, x, P.refine_sweeps, emin);
+#pragma unroll
+    for (int i = 0; i < N; i++) ks[0][i] = -x[i];
+#pragma unroll
+    for (int s = 1; s < 8; s++) {
+        const_f64_ptr row = rows + 16 * s;
+        // rows 5..7 of the tableau share their first five entries, the rest are
+        // ones: the sums of stages 6 and 7 and the solution go on from stage 5's
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            if (s >= 6) {
+                L.u[i] = L.u[i] + ks[s - 1][i];
+            } else {
+                double acc = L.uprev[i];
+#pragma unroll
+                for (int q = 0; q < s; q++) acc = fma(row[q], ks[q][i], acc);
+                L.u[i] = acc;
+            }
+        }
+        odemi_f<double>(du, L.u, L.p, fma(row[14], dt, t));
+        const double dtds = (s < 5) ? dt * row[15] : 0.0;   // rows 5..7: d = 0
+        double cq[7];
+#pragma unroll
+        for (int q = 0; q < s; q++) cq[q] = row[7 + q] * idt;
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            double acc = add_tgrad(dtds, dT[i], du[i]);
+#pragma unroll
+            for (int q = 0; q < s; q++) acc = fma(cq[q], ks[q][i], acc);
+            x[i] = acc;
+        }
+        fast_wsolve<F, N>(W, LU, x, P.refine_sweeps, emin);
+#pragma unroll
+        for (int i = 0; i < N; i++) ks[s][i] = -x[i];
+    }
+#pragma unroll
+    for (int i = 0; i < N; i++) L.u[i] = L.u[i] + ks[7][i];
+    // the error estimate is the last stage
+    const double s = fast_error_sum<N>(ks[7], L.uprev, L.u, P.abstol, P.reltol);
+    bool ok = s < 0x1p+1000;
+    if constexpr (!HW) {
+        // the pivots' and dividends' range for the quotients
+        double pmax = fabs(LU.A[0][0]), pmin = pmax;
+#pragma unroll
+        for (int i = 1; i < N; i++) {
+            pmax = fmax(pmax, fabs(LU.A[i][i]));
+            pmin = fmin(pmin, fabs(LU.A[i][i]));
+        }
+        ok = ok & (pmax < 0x1p+500) & (pmin > 0x1p-500) & (emin > -900);
+    }
+    const double EEst = fast_eest<HW, N>(s);
+    float lg;
+    const double d = fast_controller<HW>(EEst, c.erroldp, FC.att == c.nreject, kc, lg);
+    const double dtn = div_nr(dt, d);
+    if (!ok) return -1;
+    FC.att++;
+    // do_newJW: the reference reuses J right after an error rejection (here it is
+    // evaluated again, to the same values); the counter follows the reference
+    c.njacs += (c.EEst > 1.0) ? 0 : 1;
+    c.EEst = EEst;
+    if (!(d > 0.0)) {
+        c.nreject++;
+        FC.x = dtn;
+        return 0;
+    }
+    const double tn = last ? c.tf : t + dt;
+    if (tn >= FC.snext) {
+        c.tprev = t;
+        c.dt = (last && FC.att == 1) ? FC.x : dt;   // a flagged step restores the unclipped dt
+        c.t = tn;
+#pragma unroll
+        for (int r = 0; r < 3; r++)
+#pragma unroll
+            for (int i = 0; i < N; i++) {
+                double acc = 0.0;
+#pragma unroll
+                for (int q = 0; q < 8; q++) acc = fma(kRH[r][q], ks[q][i], acc);
+                L.dense[r][i] = acc;
+            }
+        rodas_savevalues(L, P, j);
+        fast_next_save(FC, c, P);
+    }
+    c.t = tn;
+#pragma unroll
+    for (int i = 0; i < N; i++) L.uprev[i] = L.u[i];
+    c.erroldp = (EEst > kc.qoldinit) ? pow_of_log2<HW>(kc.beta2, lg) : erroldp_init<HW>();
+    FC.x = fmin(dtn, c.dtmax);
+    return last ? RC_SUCCESS : 0;
+}
+// Counters between fast attempts: c.nf, nw and nsolve hold what FastCtl::att
+// does not stand for (8 evaluations and solves and one W an attempt, njacs
+// evaluations for a finite-difference time derivative).
+__device__ __forceinline__ void rodas_fast_counts(const FastCtl& F, Ctl& c, int sign) {
+    if (sign > 0) c.naccept = F.att - c.nreject;
+    c.nf += sign * (8 * F.att + (ODEMI_HAS_TGRAD ? 0 : c.njacs));
+    c.nw += sign * F.att;
+    c.nsolve += sign * 8 * F.att;
+}
+// The same attempt by the complete rules.
+template <typename F, int N>
+__device__ __forceinline__ int rodas_attempt_full(RodasLane<F, N>& L, FastCtl& FC, const Params& P, i64 j) {
+    Ctl& c = L.c;
+    rodas_fast_counts(FC, c, 1);
+    fast_to_ctl(FC, c, P);
+    if (c.accept_step) {
+#pragma unroll
+        for (int i = 0; i < N; i++) L.u[i] = L.uprev[i];
+    }
+    // J and dT for an attempt that reuses them
+#pragma unroll
+    for (int a = 0; a < N; a++)
+#pragma unroll
+        for (int b = 0; b < N; b++) L.J[a][b] = 0.0;
+    odemi_jac<double>(&L.J[0][0], L.uprev, L.p, c.t);
+    odemi_tgrad<double>(L.dT, L.uprev, L.p, c.t);
+    const int rc = rodas_attempt(L, P, j);
+    fast_from_ctl(FC, c);
+    rodas_fast_counts(FC, c, -1);
+    if (c.accept_step) {
+#pragma unroll
+        for (int i = 0; i < N; i++) L.uprev[i] = L.u[i];
+    }
+    fast_next_save(FC, c, P);
+    return rc;
+}
+
 template <typename F, int N>
 __device__ void rodas_persistent(const Params& P) {
     RodasLane<F, N> L;
     WaveQueue q;
     bool active = false, exhausted = false;
     i64 j = 0;
+    FastCtl FC;
+    const int itmax = fast_itmax(P);
+    (void)FC; (void)itmax;
     for (;;) {
         bool need = refill_now(!active && !exhausted, active);
         i64 slot = wave_fetch(&P.counters[0], q, need);
@@ -2417,6 +2718,10 @@ __device__ void rodas_persistent(const Params& P) {
             if (slot < P.N) {
                 j = P.order ? P.order[slot] : slot;
                 rodas_init(L, P, j);
+                if constexpr (kFastAttempts) {
+                    fast_init<true>(FC, L.c, P);
+                    rodas_fast_counts(FC, L.c, -1);
+                }
                 active = true;
             } else {
                 exhausted = true;
@@ -2424,8 +2729,17 @@ __device__ void rodas_persistent(const Params& P) {
         }
         if (__ballot(active) == 0) break;
         if (active) {
-            int rc = rodas_attempt(L, P, j);
+            int rc;
+            if constexpr (kFastAttempts) {
+                // until a lane of the wave ends
+                do rc = rodas_attempt_fast(L, FC, P, j, itmax);
+                while (__ballot(rc != 0) == 0);
+                if (__builtin_expect(rc < 0, 0)) rc = rodas_attempt_full(L, FC, P, j);
+            } else {
+                rc = rodas_attempt(L, P, j);
+            }
             if (rc) {
+                if constexpr (kFastAttempts) rodas_fast_counts(FC, L.c, 1);
                 finish_lane<N>(L.c, P, j, L.u, rc);
                 active = false;
             }
@@ -2631,13 +2945,39 @@ __device__ void rodas_serve_tick(const Params& P0) {
     }
 #pragma unroll
     for (int k = 0; k < ODEMI_NP; k++) L.p[k] = (k < P.np) ? P.p[(i64)k * P.N + j] : 0.0;
+    FastCtl FC;
+    const int itmax = fast_itmax(P);
+    (void)FC; (void)itmax;
+    if constexpr (kFastAttempts) {
+        if (L.c.accept_step) {   // to the state between fast attempts
+#pragma unroll
+            for (int i = 0; i < N; i++) L.uprev[i] = L.u[i];
+        }
+        fast_init<true>(FC, L.c, P);
+        rodas_fast_counts(FC, L.c, -1);
+    }
     for (int a = 0; a < P.tick_attempts; a++) {
-        int rc = rodas_attempt(L, P, j);
+        int rc;
+        if constexpr (kFastAttempts) {
+            rc = rodas_attempt_fast(L, FC, P, j, itmax);
+            if (__builtin_expect(rc < 0, 0)) rc = rodas_attempt_full(L, FC, P, j);
+        } else {
+            rc = rodas_attempt(L, P, j);
+        }
         if (rc) {
+            if constexpr (kFastAttempts) rodas_fast_counts(FC, L.c, 1);
             finish_lane<N>(L.c, P, j, L.u, rc);
             plain_store_ctl<N>(L.c, P, j, 0);
             atomicAdd(&P.req_done[P.slot_req[j]], 1ULL);
             return;
+        }
+    }
+    if constexpr (kFastAttempts) {
+        fast_to_ctl(FC, L.c, P);
+        rodas_fast_counts(FC, L.c, 1);
+        if (L.c.accept_step) {
+#pragma unroll
+            for (int i = 0; i < N; i++) L.u[i] = L.uprev[i];
         }
     }
     plain_store_ctl<N>(L.c, P, j, 1);

@@ -731,17 +731,17 @@ __device__ void wg_addsteps(const WGPtrs& S, const Params& P, const Ctl& c, int 
     for (int s = 1; s < 8; s++) {
         for (int i = tid; i < n; i += NT) {
             double acc = S.uprev[i];
-            for (int q = 0; q < s; q++) acc = acc + kRA[s][q] * ks[q * nmax + i];
+            for (int q = 0; q < s; q++) acc = acc + kRStage[s][q] * ks[q * nmax + i];
             S.fsal[i] = acc;
         }
         __syncthreads();
-        odemi_f_wg<double>(S.du, S.fsal, S.pd, t + kRc[s] * dt, n, tid, NT);
+        odemi_f_wg<double>(S.du, S.fsal, S.pd, t + kRStage[s][14] * dt, n, tid, NT);
         __syncthreads();
-        const double dtds = dt * kRd[s];
+        const double dtds = dt * kRStage[s][15];
         double* x = ks + s * nmax;
         for (int i = tid; i < n; i += NT) {
             double acc = S.du[i] + dtds * S.dT[i];
-            for (int q = 0; q < s; q++) acc = acc + (kRC[s][q] / dt) * ks[q * nmax + i];
+            for (int q = 0; q < s; q++) acc = acc + (kRStage[s][7 + q] / dt) * ks[q * nmax + i];
             x[i] = acc;
         }
         __syncthreads();
@@ -998,7 +998,7 @@ __device__ __forceinline__ int wg_run(const WGPtrs& S, const Params& P, i64 j, i
             }
             c.nw += 1;
             __syncthreads();
-            const double dtd0 = dt * kRd[0];
+            const double dtd0 = dt * kRStage[0][15];
             for (int i = tid; i < n; i += NT) ks[i] = fsal[i] + dtd0 * dT[i];
             // rb = fsal, r = du, d = u are free during the stage-1 solve
             if constexpr (GJ) {
@@ -1017,18 +1017,18 @@ __device__ __forceinline__ int wg_run(const WGPtrs& S, const Params& P, i64 j, i
             for (int s = 1; s < 8; s++) {
                 for (int i = tid; i < n; i += NT) {
                     double acc = uprev[i];
-                    for (int q = 0; q < s; q++) acc = fma(kRA[s][q], ks[q * nmax + i], acc);
+                    for (int q = 0; q < s; q++) acc = fma(kRStage[s][q], ks[q * nmax + i], acc);
                     u[i] = acc;
                 }
                 __syncthreads();
-                odemi_f_wg<double>(du, u, pp, fma(kRc[s], dt, t), n, tid, NT);
+                odemi_f_wg<double>(du, u, pp, fma(kRStage[s][14], dt, t), n, tid, NT);
                 c.nf += 1;
                 __syncthreads();
-                const double dtds = dt * kRd[s];
+                const double dtds = dt * kRStage[s][15];
                 double* x = ks + s * nmax;
                 for (int i = tid; i < n; i += NT) {
                     double acc = fma(dtds, dT[i], du[i]);
-                    for (int q = 0; q < s; q++) acc = fma(kRC[s][q] * idt, ks[q * nmax + i], acc);
+                    for (int q = 0; q < s; q++) acc = fma(kRStage[s][7 + q] * idt, ks[q * nmax + i], acc);
                     x[i] = acc;
                 }
                 __syncthreads();
@@ -1045,7 +1045,7 @@ __device__ __forceinline__ int wg_run(const WGPtrs& S, const Params& P, i64 j, i
             }
             for (int i = tid; i < n; i += NT) {
                 double acc = uprev[i];
-                for (int q = 0; q < 7; q++) acc = fma(kRA[7][q], ks[q * nmax + i], acc);
+                for (int q = 0; q < 7; q++) acc = fma(kRStage[7][q], ks[q * nmax + i], acc);
                 acc = fma(1.0, ks[7 * nmax + i], acc);
                 u[i] = acc;
                 double e = 0.0;
