@@ -13,6 +13,32 @@
 //   ODEMI_GJ_MFMA 0: one rank-1 update per step on the vector ALUs, each
 //     thread holding an R x R tile.
 #pragma once
+
+namespace odemi {
+
+// Maximum over the wave, returned to every lane.  All 64 lanes must be active.
+// Lanes without a source read 0, the identity of the unsigned maximum.
+__device__ __forceinline__ unsigned dpp_wave_max_u32(unsigned x) {
+    x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, true));
+    x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, true));
+    x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, true));
+    x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, true));
+    x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, true));  // row_bcast:15
+    x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, true));  // row_bcast:31
+    return (unsigned)__builtin_amdgcn_readlane((int)x, 63);
+}
+
+// Broadcast a value held by lane `src` (wave-uniform) to the whole wave.
+__device__ __forceinline__ float wave_bcast(float v, int src) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), src));
+}
+__device__ __forceinline__ double wave_bcast(double v, int src) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), src),
+                            __builtin_amdgcn_readlane(__double2loint(v), src));
+}
+
+}  // namespace odemi
+
 #if ODEMI_N <= 128
 #define ODEMI_GJ 1
 #define ODEMI_GJ_R ((ODEMI_N + 15) / 16)   // tile of the largest state (nmax)
@@ -41,18 +67,6 @@ __device__ __forceinline__ float dpp_row_sum16(float x) {
     x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x118, 0xf, 0xf, false));  // row_shr:8
     return x;
 }
-// Maximum over the wave, returned to every lane.  All 64 lanes must be active.
-// Lanes without a source read 0, the identity of the unsigned maximum.
-__device__ __forceinline__ unsigned dpp_wave_max_u32(unsigned x) {
-    x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, true));
-    x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, true));
-    x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, true));
-    x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, true));
-    x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, true));  // row_bcast:15
-    x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, true));  // row_bcast:31
-    return (unsigned)__builtin_amdgcn_readlane((int)x, 63);
-}
-
 __device__ __forceinline__ unsigned gj_key(float v, int i) {
     // larger |v| wins, ties to the smaller row; a NaN entry competes as zero so
     // the pivot is always an unused row < n (n <= 128)

@@ -8,18 +8,18 @@
 // is bit-identical to the restatement.
 //
 // LDS layout (dynamic, sized by the host from nmax):
-//   W    F[nmax][ld], ld = nmax + 1       J, then W = J - I/(dt*gamma), then its LU
+//   W    F[nmax][ld], ld = nmax | 1       J, then W = J - I/(dt*gamma), then its LU
 //                                         (FP64 variant only)
 //   vec  double[NV][nmax]                 u, uprev, fsal, du, dT, ks[8] (+ dense[3]);
 //   pd   double[32]                       parameters (FP64)
 //   fsc  float[nmax + 32]                 FP32 copies of uprev and p (mixed variant)
-//   piv  int[nmax], perm int[nmax]        pivots and the equivalent row gather
+//   piv  int[nmax], perm int[nmax]        row positions (scratch of the LU) and the row gather
 //   gjbuf float[51 NP + 16]               Gauss-Jordan panels, pivot rows, scales and
 //                                         mat-vec result (mixed variant; NP = 16 R,
 //                                         R = ceil(nmax/16); layout in odemi_gj.h)
 //   red  double[32] + int[32]             reductions / broadcasts
 // FP64 variant: W is FP64 in LDS (132 KB at n = 128, one workgroup per CU),
-// factored by LU with partial pivoting.
+// factored by LU with partial pivoting (odemi_lu.h).
 // Mixed variant (n <= 128): the FP32 Jacobian is evaluated into a per-workgroup
 // global scratch block, W = J - I/(dt*gamma) is held in the workgroup's
 // registers (R = ceil(n/16) per trajectory) and inverted in place by swap-free
@@ -39,6 +39,7 @@
 #define ODEMI_WG_ROWS ((ODEMI_N + 63) / 64)
 
 #include "odemi_gj.h"
+#include "odemi_lu.h"
 
 namespace odemi {
 
@@ -73,7 +74,7 @@ __host__ __device__ inline int wg_gj_floats(int nmax, bool gj) {
 template <typename F>
 __device__ __forceinline__ WGPtrs wg_layout(unsigned char* base, int nmax, bool saves, bool w_in_lds) {
     WGPtrs L;
-    L.ld = nmax + 1;
+    L.ld = nmax | 1;   // odd: a column's entries lie in different LDS banks
     size_t off = 0;
     L.W = base;
     if (w_in_lds) off += ((size_t)nmax * L.ld * sizeof(F) + 15) & ~(size_t)15;
@@ -120,18 +121,8 @@ __device__ __forceinline__ int wg_argmax(double v, int idx, double* red, int* ir
     return bi;
 }
 
-// Broadcast a value held by lane `src` (wave-uniform) to the whole wave.
-__device__ __forceinline__ float wave_bcast(float v, int src) {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), src));
-}
-__device__ __forceinline__ double wave_bcast(double v, int src) {
-    i64 b = __double_as_longlong(v);
-    int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffLL), src);
-    int hi = __builtin_amdgcn_readlane((int)(b >> 32), src);
-    return __longlong_as_double(((i64)hi << 32) | (i64)(unsigned)lo);
-}
-
-// In-place LU with partial pivoting of the n x n leading block of A (stride ld).
+// In-place LU with partial pivoting of the n x n leading block of A (stride
+// ld), element by element: the FP32 form for n > 128 (FP64: wg_lu_blocked).
 #define ODEMI_WG_CB ((ODEMI_N + 15) / 16)
 template <typename F>
 __device__ void wg_lu(F* A, int ld, int n, int* piv, int* perm, double* red, int* ired) {
@@ -191,87 +182,116 @@ __device__ void wg_lu(F* A, int ld, int n, int* piv, int* perm, double* red, int
     }
 }
 
-// x <- A^{-1} x using the LU of wg_lu.  x is FP64 in LDS; the substitutions run
-// in precision F on wave 0 (rows held in registers, the solved entry broadcast
-// with readlane), in LAPACK's column order.  All threads must call.
 template <typename F>
-__device__ void wg_lu_solve(const F* A, int ld, int n, const int* perm, double* x) {
+__device__ __forceinline__ void wg_factor(const WGPtrs& S, int n) {
+    if constexpr (sizeof(F) == sizeof(double)) wg_lu_blocked<ODEMI_WG_ROWS>((double*)S.W, S.ld, n, S.ired, S.perm);
+    else wg_lu<F>((F*)S.W, S.ld, n, S.piv, S.perm, S.red, S.ired);
+}
+
+// x <- A^{-1} x using an LU factorization, every quotient an IEEE division: the
+// FP32 form for n > 128, and the FP64 solves that wave_lu_solve declines.  x is
+// FP64 in LDS; the substitutions run in precision F on wave 0 (rows held in
+// registers, the solved entry broadcast with readlane), in LAPACK's column
+// order.  Wave 0 only.
+template <typename F>
+__device__ void wave_lu_solve_ieee(const F* A, int ld, int n, const int* perm, double* x) {
+    const int lane = threadIdx.x;
+    // row interchanges of the LU applied as one gather (same result as the
+    // sequential swaps b[k] <-> b[piv[k]], k = 0..n-1)
+    F b[ODEMI_WG_ROWS];
+#pragma unroll
+    for (int r = 0; r < ODEMI_WG_ROWS; r++) {
+        int i = lane + 64 * r;
+        b[r] = (i < n) ? (F)x[perm[i]] : (F)0;
+    }
+    // forward, unit lower triangle (column order); the solved entry is
+    // broadcast with readlane (uniform lane), the factor column is read
+    // one step ahead so the dependent chain is readlane + fma
+    F Lc[ODEMI_WG_ROWS], Ln[ODEMI_WG_ROWS];
+#pragma unroll
+    for (int r = 0; r < ODEMI_WG_ROWS; r++) {
+        int i = lane + 64 * r;
+        Lc[r] = (i < n && n > 1) ? A[i * ld + 0] : (F)0;
+    }
+    for (int c = 0; c < n - 1; c++) {
+#pragma unroll
+        for (int r = 0; r < ODEMI_WG_ROWS; r++) {
+            int i = lane + 64 * r;
+            Ln[r] = (i < n && c + 1 < n - 1) ? A[i * ld + c + 1] : (F)0;
+        }
+        F bc = b[0];
+#pragma unroll
+        for (int r = 1; r < ODEMI_WG_ROWS; r++) if ((c >> 6) == r) bc = b[r];
+        const F xc = wave_bcast(bc, c & 63);
+#pragma unroll
+        for (int r = 0; r < ODEMI_WG_ROWS; r++) {
+            int i = lane + 64 * r;
+            if (i > c && i < n) b[r] = fma(-Lc[r], xc, b[r]);
+            Lc[r] = Ln[r];
+        }
+    }
+    // backward, upper triangle (column order)
+    F Uc[ODEMI_WG_ROWS], Un[ODEMI_WG_ROWS];
+    F dc = A[(n - 1) * ld + (n - 1)], dn = (F)1;
+#pragma unroll
+    for (int r = 0; r < ODEMI_WG_ROWS; r++) {
+        int i = lane + 64 * r;
+        Uc[r] = (i < n) ? A[i * ld + (n - 1)] : (F)0;
+    }
+    for (int c = n - 1; c >= 0; c--) {
+        if (c > 0) {
+            dn = A[(c - 1) * ld + (c - 1)];
+#pragma unroll
+            for (int r = 0; r < ODEMI_WG_ROWS; r++) {
+                int i = lane + 64 * r;
+                Un[r] = (i < n) ? A[i * ld + (c - 1)] : (F)0;
+            }
+        }
+        F bc = b[0];
+#pragma unroll
+        for (int r = 1; r < ODEMI_WG_ROWS; r++) if ((c >> 6) == r) bc = b[r];
+        const F xc = wave_bcast(bc, c & 63) / dc;
+#pragma unroll
+        for (int r = 0; r < ODEMI_WG_ROWS; r++) {
+            int i = lane + 64 * r;
+            if (i == c) b[r] = xc;
+            else if (i < c) b[r] = fma(-Uc[r], xc, b[r]);
+            Uc[r] = Un[r];
+        }
+        dc = dn;
+    }
+#pragma unroll
+    for (int r = 0; r < ODEMI_WG_ROWS; r++) {
+        int i = lane + 64 * r;
+        if (i < n) x[i] = (double)b[r];
+    }
+}
+
+// x <- A^{-1} x with the factors of wg_lu (FP32) or wg_lu_blocked (FP64, negated
+// if NEG).  All threads must call.
+template <typename F, bool NEG>
+__device__ __forceinline__ void wg_lu_solve(const F* A, int ld, int n, const int* perm, double* x) {
     if (threadIdx.x < 64) {
-        const int lane = threadIdx.x;
-        // row interchanges of the LU applied as one gather (same result as the
-        // sequential swaps b[k] <-> b[piv[k]], k = 0..n-1)
-        F b[ODEMI_WG_ROWS];
-#pragma unroll
-        for (int r = 0; r < ODEMI_WG_ROWS; r++) {
-            int i = lane + 64 * r;
-            b[r] = (i < n) ? (F)x[perm[i]] : (F)0;
-        }
-        // forward, unit lower triangle (column order); the solved entry is
-        // broadcast with readlane (uniform lane), the factor column is read
-        // one step ahead so the dependent chain is readlane + fma
-        F Lc[ODEMI_WG_ROWS], Ln[ODEMI_WG_ROWS];
-#pragma unroll
-        for (int r = 0; r < ODEMI_WG_ROWS; r++) {
-            int i = lane + 64 * r;
-            Lc[r] = (i < n && n > 1) ? A[i * ld + 0] : (F)0;
-        }
-        for (int c = 0; c < n - 1; c++) {
-#pragma unroll
-            for (int r = 0; r < ODEMI_WG_ROWS; r++) {
-                int i = lane + 64 * r;
-                Ln[r] = (i < n && c + 1 < n - 1) ? A[i * ld + c + 1] : (F)0;
+        if constexpr (sizeof(F) == sizeof(double)) {
+            if (!wave_lu_solve<ODEMI_WG_ROWS, NEG>(A, ld, n, perm, x)) {
+                wave_lu_solve_ieee<F>(A, ld, n, perm, x);
+                if (NEG)
+                    for (int i = threadIdx.x; i < n; i += 64) x[i] = -x[i];
             }
-            F bc = b[0];
-#pragma unroll
-            for (int r = 1; r < ODEMI_WG_ROWS; r++) if ((c >> 6) == r) bc = b[r];
-            const F xc = wave_bcast(bc, c & 63);
-#pragma unroll
-            for (int r = 0; r < ODEMI_WG_ROWS; r++) {
-                int i = lane + 64 * r;
-                if (i > c && i < n) b[r] = fma(-Lc[r], xc, b[r]);
-                Lc[r] = Ln[r];
-            }
-        }
-        // backward, upper triangle (column order)
-        F Uc[ODEMI_WG_ROWS], Un[ODEMI_WG_ROWS];
-        F dc = A[(n - 1) * ld + (n - 1)], dn = (F)1;
-#pragma unroll
-        for (int r = 0; r < ODEMI_WG_ROWS; r++) {
-            int i = lane + 64 * r;
-            Uc[r] = (i < n) ? A[i * ld + (n - 1)] : (F)0;
-        }
-        for (int c = n - 1; c >= 0; c--) {
-            if (c > 0) {
-                dn = A[(c - 1) * ld + (c - 1)];
-#pragma unroll
-                for (int r = 0; r < ODEMI_WG_ROWS; r++) {
-                    int i = lane + 64 * r;
-                    Un[r] = (i < n) ? A[i * ld + (c - 1)] : (F)0;
-                }
-            }
-            F bc = b[0];
-#pragma unroll
-            for (int r = 1; r < ODEMI_WG_ROWS; r++) if ((c >> 6) == r) bc = b[r];
-            const F xc = wave_bcast(bc, c & 63) / dc;
-#pragma unroll
-            for (int r = 0; r < ODEMI_WG_ROWS; r++) {
-                int i = lane + 64 * r;
-                if (i == c) b[r] = xc;
-                else if (i < c) b[r] = fma(-Uc[r], xc, b[r]);
-                Uc[r] = Un[r];
-            }
-            dc = dn;
-        }
-#pragma unroll
-        for (int r = 0; r < ODEMI_WG_ROWS; r++) {
-            int i = lane + 64 * r;
-            if (i < n) x[i] = (double)b[r];
+        } else {
+            static_assert(!NEG, "the FP32 solution is refined before its sign changes");
+            wave_lu_solve_ieee<F>(A, ld, n, perm, x);
         }
     }
     __syncthreads();
 }
 
-// Stage solve W x = b (b in `x` on entry; x must be visible to all threads).
+__device__ __forceinline__ void wg_negate(double* x, int n) {
+    for (int i = threadIdx.x; i < n; i += blockDim.x) x[i] = -x[i];
+    __syncthreads();
+}
+
+// Stage solve, x <- -W^{-1} x (x must be visible to all threads).
 // FP64: one LU solve.  Mixed: FP32 LU solve plus refinement sweeps with the
 // FP64 residual r = b - J x + sigma x (J x from the traced Jacobian-vector
 // product at uprev).  Scratch: rb (copy of b), r, d -- three free vectors.
@@ -280,26 +300,27 @@ __device__ void wg_wsolve(const WGPtrs& S, int n, double* x, double* rb, double*
                           const double* uprev, const double* p, double t, double sigma, int sweeps) {
     const F* A = (const F*)S.W;
     if constexpr (sizeof(F) == sizeof(double)) {
-        wg_lu_solve<F>(A, S.ld, n, S.perm, x);
+        wg_lu_solve<F, true>(A, S.ld, n, S.perm, x);
     } else {
         const int tid = threadIdx.x, NT = blockDim.x;
         for (int i = tid; i < n; i += NT) rb[i] = x[i];
         __syncthreads();
-        wg_lu_solve<F>(A, S.ld, n, S.perm, x);
+        wg_lu_solve<F, false>(A, S.ld, n, S.perm, x);
         for (int sw = 0; sw < sweeps; sw++) {
             odemi_jvp_wg<double>(r, x, uprev, p, t, n, tid, NT);
             __syncthreads();
             for (int i = tid; i < n; i += NT) d[i] = fma(sigma, x[i], rb[i] - r[i]);
             __syncthreads();
-            wg_lu_solve<F>(A, S.ld, n, S.perm, d);
-            for (int i = tid; i < n; i += NT) x[i] = x[i] + d[i];
+            wg_lu_solve<F, false>(A, S.ld, n, S.perm, d);
+            for (int i = tid; i < n; i += NT) x[i] = (sw + 1 < sweeps) ? x[i] + d[i] : -(x[i] + d[i]);
             __syncthreads();
         }
+        if (sweeps <= 0) wg_negate(x, n);
     }
 }
 
 #if ODEMI_GJ
-// Stage solve W x = b for the Gauss-Jordan variant (b in x on entry), with the
+// Stage solve, x <- -W^{-1} x, for the Gauss-Jordan variant, with the
 // same FP64 refinement sweeps as wg_wsolve.  gjbuf holds gj_invert<R>'s
 // buffers (sized for the largest R), zbuf at gj_zbuf_off<R>().
 template <int R>
@@ -316,9 +337,10 @@ __device__ __forceinline__ void wg_wsolve_gj(const GJTile<R>& G, const WGPtrs& S
         for (int i = tid; i < n; i += NT) d[i] = fma(sigma, x[i], rb[i] - r[i]);
         __syncthreads();
         gj_solve<R>(G, n, S.perm, d, zbuf);
-        for (int i = tid; i < n; i += NT) x[i] = x[i] + d[i];
+        for (int i = tid; i < n; i += NT) x[i] = (sw + 1 < sweeps) ? x[i] + d[i] : -(x[i] + d[i]);
         __syncthreads();
     }
+    if (sweeps <= 0) wg_negate(x, n);
 }
 #endif  // ODEMI_GJ
 
@@ -333,6 +355,22 @@ __device__ __forceinline__ void wg_save_point(Ctl& c, double& tlast, const Param
     tlast = t;
 }
 
+// sum of v[i]^2 as the index-order fma chain, eight loads ahead of it
+__device__ __forceinline__ double wg_sum_squares(const double* v, int n) {
+    double s = 0.0, x[8], y[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) x[j] = v[min(j, n - 1)];
+    for (int i = 0; i < n; i += 8) {
+#pragma unroll
+        for (int j = 0; j < 8; j++) y[j] = v[min(i + 8 + j, n - 1)];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            if (i + j < n) s = fma(x[j], x[j], s);
+            x[j] = y[j];
+        }
+    }
+    return s;
+}
 // Index-order fma-chain norms, evaluated by one thread (bit-identical to the
 // sequential restatement).
 __device__ __forceinline__ double wg_norm_div(const double* a, const double* sk, int n) {
@@ -458,6 +496,25 @@ __device__ __forceinline__ void wg_begin(const WGPtrs& S, const Params& P, i64 j
 #else
 #define ODEMI_WG_EVENTS 0
 #endif
+
+// acc + sum over q < s of coef[q] (times idt if SCALE) k[q * nmax], as an fma
+// chain.  AHEAD: coefficients and stage values of every q are loaded before the
+// chain instead of one by one in it (about 1,000 cycles a sum); the mixed kernel
+// has no registers left for them.
+template <bool AHEAD, bool SCALE>
+__device__ __forceinline__ double wg_stage_sum(double acc, const_f64_ptr coef, double idt, const double* k, int nmax,
+                                               int s) {
+    if constexpr (AHEAD) {
+        double a[7], v[7];
+#pragma unroll
+        for (int q = 0; q < 7; q++) { a[q] = SCALE ? coef[q] * idt : coef[q]; v[q] = k[q * nmax]; }
+#pragma unroll
+        for (int q = 0; q < 7; q++) acc = (q < s) ? fma(a[q], v[q], acc) : acc;
+    } else {
+        for (int q = 0; q < s; q++) acc = fma(SCALE ? coef[q] * idt : coef[q], k[q * nmax], acc);
+    }
+    return acc;
+}
 
 #ifdef ODEMI_WG_CALLBACKS
 // ---------------------------------------------------------------------------
@@ -713,7 +770,7 @@ __device__ void wg_addsteps(const WGPtrs& S, const Params& P, const Ctl& c, int 
         __syncthreads();
         for (int i = tid; i < n; i += NT) W[i * ld + i] = (F)fma(-1.0, sigma, (double)W[i * ld + i]);
         __syncthreads();
-        wg_lu<F>(W, ld, n, S.piv, S.perm, S.red, S.ired);
+        wg_factor<F>(S, n);
     }
     __syncthreads();
     auto solve = [&](double* x) {
@@ -724,8 +781,6 @@ __device__ void wg_addsteps(const WGPtrs& S, const Params& P, const Ctl& c, int 
         } else {
             wg_wsolve<F>(S, n, x, sc0, sc1, sc2, S.uprev, S.pd, t, sigma, P.refine_sweeps);
         }
-        for (int i = tid; i < n; i += NT) x[i] = -x[i];
-        __syncthreads();
     };
     solve(ks);
     for (int s = 1; s < 8; s++) {
@@ -1008,29 +1063,21 @@ __device__ __forceinline__ int wg_run(const WGPtrs& S, const Params& P, i64 j, i
                 wg_wsolve_gj<R>(G, S, n, ks, fsal, du, u, uprev, pp, t, sigma, P.refine_sweeps);
 #endif
             } else {
-                wg_lu<F>(W, ld, n, S.piv, S.perm, red, S.ired);
+                wg_factor<F>(S, n);
                 wg_wsolve<F>(S, n, ks, fsal, du, u, uprev, pp, t, sigma, P.refine_sweeps);
             }
-            for (int i = tid; i < n; i += NT) ks[i] = -ks[i];
             c.nsolve += 1;
-            __syncthreads();
             for (int s = 1; s < 8; s++) {
-                for (int i = tid; i < n; i += NT) {
-                    double acc = uprev[i];
-                    for (int q = 0; q < s; q++) acc = fma(kRStage[s][q], ks[q * nmax + i], acc);
-                    u[i] = acc;
-                }
+                const const_f64_ptr row = (const_f64_ptr)(&kRStage[0][0]) + 16 * s;
+                const double ct = row[14], dtds = dt * row[15];
+                for (int i = tid; i < n; i += NT) u[i] = wg_stage_sum<!GJ, false>(uprev[i], row, idt, ks + i, nmax, s);
                 __syncthreads();
-                odemi_f_wg<double>(du, u, pp, fma(kRStage[s][14], dt, t), n, tid, NT);
+                odemi_f_wg<double>(du, u, pp, fma(ct, dt, t), n, tid, NT);
                 c.nf += 1;
                 __syncthreads();
-                const double dtds = dt * kRStage[s][15];
                 double* x = ks + s * nmax;
-                for (int i = tid; i < n; i += NT) {
-                    double acc = fma(dtds, dT[i], du[i]);
-                    for (int q = 0; q < s; q++) acc = fma(kRStage[s][7 + q] * idt, ks[q * nmax + i], acc);
-                    x[i] = acc;
-                }
+                for (int i = tid; i < n; i += NT)
+                    x[i] = wg_stage_sum<!GJ, true>(fma(dtds, dT[i], du[i]), row + 7, idt, ks + i, nmax, s);
                 __syncthreads();
                 if constexpr (GJ) {
 #if ODEMI_GJ
@@ -1039,9 +1086,7 @@ __device__ __forceinline__ int wg_run(const WGPtrs& S, const Params& P, i64 j, i
                 } else {
                     wg_wsolve<F>(S, n, x, fsal, du, u, uprev, pp, t, sigma, P.refine_sweeps);
                 }
-                for (int i = tid; i < n; i += NT) x[i] = -x[i];
                 c.nsolve += 1;
-                __syncthreads();
             }
             for (int i = tid; i < n; i += NT) {
                 double acc = uprev[i];
@@ -1068,8 +1113,7 @@ __device__ __forceinline__ int wg_run(const WGPtrs& S, const Params& P, i64 j, i
                 fsal[i] = du[i] / fma(max_fast(fabs(uprev[i]), fabs(u[i])), P.reltol, P.abstol);
             __syncthreads();
             if (tid == 0) {
-                double sq = 0.0;
-                for (int i = 0; i < n; i++) sq = fma(fsal[i], fsal[i], sq);
+                const double sq = wg_sum_squares(fsal, n);
                 red[24] = sqrt(sq / (double)(n > 1 ? n : 1));
             }
             __syncthreads();

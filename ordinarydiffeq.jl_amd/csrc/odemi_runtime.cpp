@@ -688,7 +688,7 @@ size_t gj_ld(int nmax) { return 16 * (((size_t)nmax + 15) / 16); }
 
 // Dynamic LDS of the workgroup kernels; must match odemi::wg_layout in kernels/odemi_wg.h.
 size_t wg_shmem_bytes(int nmax, bool mixed, bool saves, bool gj) {
-    const size_t ld = (size_t)nmax + 1, fb = mixed ? 4 : 8;
+    const size_t ld = (size_t)nmax | 1, fb = mixed ? 4 : 8;
     const size_t np16 = 16 * (((size_t)nmax + 15) / 16);
     size_t shmem = gj ? 0 : (((size_t)nmax * ld * fb + 15) & ~(size_t)15);
     shmem += (size_t)(13 + (saves ? 3 : 0)) * nmax * 8 + 32 * 8;  // vectors + parameters (<= 32)
