@@ -1111,10 +1111,14 @@ double now_s() {
 
 struct Request {
     int64_t id = 0, N = 0;
-    std::vector<double> u0, p, t0, tf;   // host copies of the inputs (SoA, N columns)
-    std::vector<double> tol;             // reltol [N] then abstol [N] (the request's own or the server's)
+    // copy of the inputs (SoA, N columns): in the server's pinned ring from `src`
+    // on (u0, p, t0, tf, then nvec), or, without room there, in the vectors
+    const double* src = nullptr;
+    std::vector<double> u0, p, t0, tf;
     std::vector<int> nvec;               // per-trajectory n (workgroup servers)
-    std::vector<int> sreq;               // slot -> request-table index for the admitted range
+    std::vector<double> tol;             // reltol [N] then abstol [N] (vectors only)
+    std::vector<int> sreq;               // slot -> request-table index for the admitted range (vectors only)
+    double reltol = 0, abstol = 0;       // the request's own or the server's
     double* u_final = nullptr;           // caller's output buffers
     int32_t* retcode = nullptr;
     int32_t* stats = nullptr;
@@ -1159,6 +1163,90 @@ struct RangeAlloc {
         if (last->first + last->second >= high) high = std::min(high, last->first);
     }
 };
+
+// Ring of pinned host memory for the inputs of requests not yet admitted.
+// Ranges are taken in submission order and given back in any order; a range
+// in front of the oldest one still held becomes free.
+struct PinnedRing {
+    struct Range { size_t off; bool held; };
+    char* base = nullptr;
+    size_t cap = 0, head = 0;
+    std::deque<Range> q;
+    void* take(size_t len) {
+        len = (len + 255) & ~size_t(255);
+        if (q.empty()) head = 0;
+        size_t off;
+        if (q.empty() || head > q.front().off) {
+            if (cap - head >= len) off = head;
+            else if (!q.empty() && q.front().off > len) off = 0;
+            else return nullptr;
+        } else {
+            if (q.front().off - head <= len) return nullptr;   // never head == front while a range is held
+            off = head;
+        }
+        q.push_back({off, true});
+        head = off + len;
+        return base + off;
+    }
+    void give(const void* p) {
+        const size_t off = (size_t)((const char*)p - base);
+        for (auto& r : q)
+            if (r.off == off) r.held = false;
+        while (!q.empty() && !q.front().held) q.pop_front();
+    }
+};
+
+// One request's inputs into its slots, or its results out of them.  Both
+// kernels read or write pinned host memory in place: a burst of requests is one
+// launch each way, where a copy of every array of every request (ten small
+// pageable copies, two fills and a launch each, ~200 us a request) had been the
+// time of a serving burst.
+struct AdmitEntry {
+    const double* src;
+    int64_t slot0, N;
+    double reltol, abstol;
+    int rt, pad;
+};
+struct ResultEntry {
+    double* u;
+    int *rc, *st;
+    int64_t slot0, N;
+};
+__global__ void __launch_bounds__(256) serve_admit_kernel(Params P, const AdmitEntry* tab, int n, int np, int wg) {
+    const AdmitEntry e = tab[blockIdx.y];
+    const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (k >= e.N) return;
+    const int64_t s = e.slot0 + k, S = P.N, N = e.N;
+    const double* src = e.src + k;
+    for (int r = 0; r < n; r++) ((double*)P.u0)[r * S + s] = src[r * N];
+    src += n * N;
+    for (int r = 0; r < np; r++) ((double*)P.p)[r * S + s] = src[r * N];
+    if (np == 0) ((double*)P.p)[s] = 0.0;
+    src += np * N;
+    ((double*)P.t0)[s] = src[0];
+    ((double*)P.tf)[s] = src[N];
+    if (wg) ((int*)P.nvec)[s] = ((const int*)(e.src + (n + np + 2) * N))[k];
+    // the slots' tolerances: scalar state rows 10 (reltol) and 11 (abstol)
+    P.st_scalar[10 * S + s] = e.reltol;
+    P.st_scalar[11 * S + s] = e.abstol;
+    ((int*)P.slot_req)[s] = e.rt;
+    P.nsaved[s] = 0;
+    if (k == 0) P.req_done[e.rt] = 0;
+}
+__global__ void __launch_bounds__(256) serve_result_kernel(Params P, const ResultEntry* tab, int n) {
+    const ResultEntry e = tab[blockIdx.y];
+    const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (k >= e.N) return;
+    const int64_t s = e.slot0 + k, S = P.N, N = e.N;
+    for (int r = 0; r < n; r++) e.u[r * N + k] = P.u_final[r * S + s];
+    e.rc[k] = P.retcode[s];
+    for (int r = 0; r < (int)kStatRows; r++) e.st[r * N + k] = P.stats[r * S + s];
+}
+__global__ void __launch_bounds__(256) serve_done_kernel(const unsigned long long* done, unsigned long long* host, int m) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < m) host[i] = done[i];
+}
+constexpr size_t kRingBytes = 8 << 20, kResultBytes = 4 << 20;
 }  // namespace
 
 struct odemi_server {
@@ -1174,7 +1262,13 @@ struct odemi_server {
     hipStream_t stream = nullptr;
     void* mem = nullptr;
     Params P;
-    std::vector<unsigned long long> done_h;
+    // pinned host memory: completion counts, kernel tables, result staging, input ring
+    void* pinned = nullptr;
+    unsigned long long* done_h = nullptr;
+    AdmitEntry* admit_tab = nullptr;
+    ResultEntry* result_tab = nullptr;
+    char* result_buf = nullptr;
+    PinnedRing ring;
     RangeAlloc alloc;
     std::vector<int> rt_free;
     std::mutex mu;
@@ -1303,11 +1397,23 @@ extern "C" odemi_server* odemi_server_create(odemi_ctx* ctx, odemi_rhs* rhs, con
     }
     P.refine_sweeps = opts->refine_sweeps;
     P.tick_attempts = opts->tick_attempts > 0 ? opts->tick_attempts : 64;
-    S->done_h.assign(S->R, 0);
+    const size_t b_done = (size_t)S->R * 8, b_admit = (size_t)S->R * sizeof(AdmitEntry),
+                 b_result = (size_t)S->R * sizeof(ResultEntry);
+    if (hipHostMalloc(&S->pinned, b_done + b_admit + b_result + kResultBytes + kRingBytes, hipHostMallocDefault) != hipSuccess) {
+        ctx->err = "pinned host memory allocation failed"; (void)hipFree(S->mem); delete S; return nullptr;
+    }
+    char* hp = (char*)S->pinned;
+    S->done_h = (unsigned long long*)hp;
+    S->admit_tab = (AdmitEntry*)(hp + b_done);
+    S->result_tab = (ResultEntry*)(hp + b_done + b_admit);
+    S->result_buf = hp + b_done + b_admit + b_result;
+    S->ring.base = S->result_buf + kResultBytes;
+    S->ring.cap = kRingBytes;
+    memset(S->done_h, 0, b_done);
     S->alloc = RangeAlloc(slots);
     for (int i = S->R - 1; i >= 0; i--) S->rt_free.push_back(i);
     if (hipStreamCreateWithFlags(&S->stream, hipStreamNonBlocking) != hipSuccess) {
-        ctx->err = "stream create failed"; (void)hipFree(S->mem); delete S; return nullptr;
+        ctx->err = "stream create failed"; (void)hipHostFree(S->pinned); (void)hipFree(S->mem); delete S; return nullptr;
     }
     S->worker = std::thread(server_loop, S);
     return S;
@@ -1333,6 +1439,7 @@ extern "C" void odemi_server_destroy(odemi_server* S) {
     (void)hipStreamSynchronize(S->stream);
     (void)hipStreamDestroy(S->stream);
     (void)hipFree(S->mem);
+    (void)hipHostFree(S->pinned);
     for (auto& kv : S->all) delete kv.second;
     delete S;
 }
@@ -1362,28 +1469,15 @@ extern "C" int64_t odemi_submit_opts(odemi_server* S, int64_t N, const int32_t* 
     if (S->rhs->np > 0 && !p) { S->err = "the problem has parameters but p is NULL"; return -1; }
     if (N > S->S) { S->err = "request larger than the slot pool"; return -2; }
     const int n = S->rhs->n, np = S->rhs->np;
+    if (nvec)
+        for (int64_t k = 0; k < N; k++) {
+            if (S->wg && (nvec[k] < 1 || nvec[k] > n)) { S->err = "nvec entries must lie in [1, n]"; return -3; }
+            if (!S->wg && nvec[k] != n) { S->err = "uneven nvec needs a workgroup (Rodas5P) server"; return -3; }
+        }
     Request* r = new Request();
     r->N = N;
-    r->u0.assign(u0, u0 + (size_t)n * N);
-    if (np > 0 && p) r->p.assign(p, p + (size_t)np * N); else r->p.assign((size_t)std::max(np, 1) * N, 0.0);
-    r->t0.assign(t0, t0 + N);
-    r->tf.assign(tf, tf + N);
-    const double rt = (ro && ro->reltol > 0.0) ? ro->reltol : S->o.reltol;
-    const double at = (ro && ro->abstol > 0.0) ? ro->abstol : S->o.abstol;
-    r->tol.assign((size_t)2 * N, rt);
-    std::fill(r->tol.begin() + N, r->tol.end(), at);
-    if (S->wg) {
-        r->nvec.assign(N, n);
-        if (nvec) {
-            for (int64_t k = 0; k < N; k++) {
-                if (nvec[k] < 1 || nvec[k] > n) { S->err = "nvec entries must lie in [1, n]"; delete r; return -3; }
-                r->nvec[k] = nvec[k];
-            }
-        }
-    } else if (nvec) {
-        for (int64_t k = 0; k < N; k++)
-            if (nvec[k] != n) { S->err = "uneven nvec needs a workgroup (Rodas5P) server"; delete r; return -3; }
-    }
+    r->reltol = (ro && ro->reltol > 0.0) ? ro->reltol : S->o.reltol;
+    r->abstol = (ro && ro->abstol > 0.0) ? ro->abstol : S->o.abstol;
     r->u_final = u_final; r->retcode = retcode; r->stats = stats;
     if (ro) {
         const bool saves = ro->t_out != nullptr;
@@ -1425,9 +1519,42 @@ extern "C" int64_t odemi_submit_opts(odemi_server* S, int64_t N, const int32_t* 
         r->ropt[4] = -1;
     }
     r->t_submit = now_s();
+    // inputs up to 1 MiB go to the pinned ring while it has room
+    const size_t need = (size_t)N * (n + np + 2) * 8 + (S->wg ? (size_t)N * 4 : 0);
+    double* src = nullptr;
+    if (need <= ((size_t)1 << 20)) {
+        std::lock_guard<std::mutex> lk(S->mu);
+        src = (double*)S->ring.take(need);
+    }
+    if (src) {
+        memcpy(src, u0, (size_t)n * N * 8);
+        if (np > 0) memcpy(src + (size_t)n * N, p, (size_t)np * N * 8);
+        memcpy(src + (size_t)(n + np) * N, t0, (size_t)N * 8);
+        memcpy(src + (size_t)(n + np + 1) * N, tf, (size_t)N * 8);
+        if (S->wg) {
+            int* nv = (int*)(src + (size_t)(n + np + 2) * N);
+            for (int64_t k = 0; k < N; k++) nv[k] = nvec ? nvec[k] : n;
+        }
+        r->src = src;
+    } else {
+        r->u0.assign(u0, u0 + (size_t)n * N);
+        if (np > 0) r->p.assign(p, p + (size_t)np * N); else r->p.assign((size_t)N, 0.0);
+        r->t0.assign(t0, t0 + N);
+        r->tf.assign(tf, tf + N);
+        r->tol.assign((size_t)2 * N, r->reltol);
+        std::fill(r->tol.begin() + N, r->tol.end(), r->abstol);
+        if (S->wg) {
+            if (nvec) r->nvec.assign(nvec, nvec + N); else r->nvec.assign(N, n);
+        }
+    }
     {
         std::lock_guard<std::mutex> lk(S->mu);
-        if (S->stop) { S->err = "the server has stopped"; delete r; return -4; }
+        if (S->stop) {
+            S->err = "the server has stopped";
+            if (src) S->ring.give(src);
+            delete r;
+            return -4;
+        }
         r->id = S->next_id++;
         S->all[r->id] = r;
         S->pending.push_back(r);
@@ -1514,6 +1641,7 @@ static void server_loop(odemi_server* S) {
     for (;;) {
         std::vector<Request*> admit;
         int64_t high = 0;
+        int nrt = 0;   // request-table entries in use lie below it
         {
             std::unique_lock<std::mutex> lk(S->mu);
             S->cv.wait(lk, [&] { return S->stop || !S->pending.empty() || !S->active.empty(); });
@@ -1535,19 +1663,31 @@ static void server_loop(odemi_server* S) {
                 S->admitted++;
             }
             high = S->alloc.high;
+            for (const Request* r : S->active) nrt = std::max(nrt, r->rt + 1);
         }
+        int nring = 0;
+        int64_t nmost = 0;
         for (Request* r : admit) {
             const size_t N = (size_t)r->N, s0 = (size_t)r->slot0;
-            SCHK(hipMemcpy2DAsync((double*)S->P.u0 + s0, Sz * 8, r->u0.data(), N * 8, N * 8, n, hipMemcpyHostToDevice, S->stream));
-            SCHK(hipMemcpy2DAsync((double*)S->P.p + s0, Sz * 8, r->p.data(), N * 8, N * 8, np, hipMemcpyHostToDevice, S->stream));
-            SCHK(hipMemcpyAsync((double*)S->P.t0 + s0, r->t0.data(), N * 8, hipMemcpyHostToDevice, S->stream));
-            SCHK(hipMemcpyAsync((double*)S->P.tf + s0, r->tf.data(), N * 8, hipMemcpyHostToDevice, S->stream));
-            // the slots' tolerances: scalar state rows 10 (reltol) and 11 (abstol)
-            SCHK(hipMemcpyAsync(S->P.st_scalar + 10 * Sz + s0, r->tol.data(), N * 8, hipMemcpyHostToDevice, S->stream));
-            SCHK(hipMemcpyAsync(S->P.st_scalar + 11 * Sz + s0, r->tol.data() + N, N * 8, hipMemcpyHostToDevice,
-                                S->stream));
-            r->sreq.assign(N, r->rt);
-            SCHK(hipMemcpyAsync((int*)S->P.slot_req + s0, r->sreq.data(), N * 4, hipMemcpyHostToDevice, S->stream));
+            if (r->src) {
+                S->admit_tab[nring++] = {r->src, r->slot0, r->N, r->reltol, r->abstol, r->rt, 0};
+                nmost = std::max(nmost, r->N);
+            } else {
+                SCHK(hipMemcpy2DAsync((double*)S->P.u0 + s0, Sz * 8, r->u0.data(), N * 8, N * 8, n, hipMemcpyHostToDevice, S->stream));
+                SCHK(hipMemcpy2DAsync((double*)S->P.p + s0, Sz * 8, r->p.data(), N * 8, N * 8, np, hipMemcpyHostToDevice, S->stream));
+                SCHK(hipMemcpyAsync((double*)S->P.t0 + s0, r->t0.data(), N * 8, hipMemcpyHostToDevice, S->stream));
+                SCHK(hipMemcpyAsync((double*)S->P.tf + s0, r->tf.data(), N * 8, hipMemcpyHostToDevice, S->stream));
+                // the slots' tolerances: scalar state rows 10 (reltol) and 11 (abstol)
+                SCHK(hipMemcpyAsync(S->P.st_scalar + 10 * Sz + s0, r->tol.data(), N * 8, hipMemcpyHostToDevice, S->stream));
+                SCHK(hipMemcpyAsync(S->P.st_scalar + 11 * Sz + s0, r->tol.data() + N, N * 8, hipMemcpyHostToDevice,
+                                    S->stream));
+                r->sreq.assign(N, r->rt);
+                SCHK(hipMemcpyAsync((int*)S->P.slot_req + s0, r->sreq.data(), N * 4, hipMemcpyHostToDevice, S->stream));
+                SCHK(hipMemsetAsync(S->P.req_done + r->rt, 0, 8, S->stream));
+                SCHK(hipMemsetAsync((int*)S->P.nsaved + s0, 0, N * 4, S->stream));
+                if (S->wg) SCHK(hipMemcpyAsync((int*)S->P.nvec + s0, r->nvec.data(), N * 4, hipMemcpyHostToDevice, S->stream));
+                // the host input vectors live in the Request until it finishes, so no wait here
+            }
             if (S->P.req_opts) {   // the request's save / stopping times and flags
                 if (!r->sa.empty())
                     SCHK(hipMemcpyAsync((double*)S->P.req_saveat + (size_t)r->rt * S->P.sa_cap, r->sa.data(),
@@ -1558,19 +1698,27 @@ static void server_loop(odemi_server* S) {
                 SCHK(hipMemcpyAsync((int*)S->P.req_opts + (size_t)r->rt * kReqOpts, r->ropt,
                                     sizeof(r->ropt), hipMemcpyHostToDevice, S->stream));
             }
-            SCHK(hipMemsetAsync(S->P.req_done + r->rt, 0, 8, S->stream));
-            SCHK(hipMemsetAsync((int*)S->P.nsaved + s0, 0, N * 4, S->stream));
-            if (S->wg) SCHK(hipMemcpyAsync((int*)S->P.nvec + s0, r->nvec.data(), N * 4, hipMemcpyHostToDevice, S->stream));
+        }
+        if (nring > 0) {
+            hipLaunchKernelGGL(serve_admit_kernel, dim3((unsigned)((nmost + 255) / 256), (unsigned)nring), dim3(256), 0,
+                               S->stream, S->P, (const AdmitEntry*)S->admit_tab, n, S->rhs->np, S->wg ? 1 : 0);
+            SCHK(hipGetLastError());
+        }
+        // start-up work of the admitted slots, one launch per run of neighbours
+        std::sort(admit.begin(), admit.end(), [](const Request* a, const Request* b) { return a->slot0 < b->slot0; });
+        for (size_t i = 0; i < admit.size();) {
+            const int64_t s0 = admit[i]->slot0;
+            int64_t N = 0;
+            while (i < admit.size() && admit[i]->slot0 == s0 + N) N += admit[i++]->N;
             Params Pi = S->P;
-            Pi.slot0 = (int64_t)s0;
-            Pi.nslots = (int64_t)N;
+            Pi.slot0 = s0;
+            Pi.nslots = N;
             void* args[] = {&Pi};
             if (S->wg)   // one workgroup per admitted slot
-                SCHK(hipModuleLaunchKernel(f_init, (unsigned)std::min<size_t>(N, (size_t)S->wg_grid), 1, 1, 256, 1, 1,
+                SCHK(hipModuleLaunchKernel(f_init, (unsigned)std::min<int64_t>(N, S->wg_grid), 1, 1, 256, 1, 1,
                                            (unsigned)S->shmem, S->stream, args, nullptr));
             else
                 SCHK(hipModuleLaunchKernel(f_init, (unsigned)((N + 255) / 256), 1, 1, 256, 1, 1, 0, S->stream, args, nullptr));
-            // the host input vectors live in the Request until it finishes, so no wait here
         }
         if (high > 0 && S->wg) {
             // workgroups take slots of [0, high) from counters[0]
@@ -1586,12 +1734,18 @@ static void server_loop(odemi_server* S) {
             void* args[] = {&Pt};
             SCHK(hipModuleLaunchKernel(f_tick, (unsigned)((high + 255) / 256), 1, 1, 256, 1, 1, 0, S->stream, args, nullptr));
         }
-        SCHK(hipMemcpyAsync(S->done_h.data(), S->P.req_done, (size_t)S->R * 8, hipMemcpyDeviceToHost, S->stream));
+        if (nrt > 0) {
+            hipLaunchKernelGGL(serve_done_kernel, dim3((unsigned)((nrt + 255) / 256)), dim3(256), 0, S->stream,
+                               (const unsigned long long*)S->P.req_done, S->done_h, nrt);
+            SCHK(hipGetLastError());
+        }
         SCHK(hipStreamSynchronize(S->stream));
         std::vector<Request*> fin;
         {
             std::lock_guard<std::mutex> lk(S->mu);
             S->ticks++;
+            for (Request* r : admit)
+                if (r->src) { S->ring.give(r->src); r->src = nullptr; }
             for (size_t i = 0; i < S->active.size();) {
                 Request* r = S->active[i];
                 if ((int64_t)S->done_h[r->rt] >= r->N) {
@@ -1603,22 +1757,52 @@ static void server_loop(odemi_server* S) {
                 }
             }
         }
-        for (Request* r : fin) {
-            const size_t N = (size_t)r->N, s0 = (size_t)r->slot0;
-            if (r->u_final)
-                SCHK(hipMemcpy2DAsync(r->u_final, N * 8, (double*)S->P.u_final + s0, Sz * 8, N * 8, n, hipMemcpyDeviceToHost, S->stream));
-            SCHK(hipMemcpyAsync(r->retcode, (int*)S->P.retcode + s0, N * 4, hipMemcpyDeviceToHost, S->stream));
-            if (r->stats)
-                SCHK(hipMemcpy2DAsync(r->stats, N * 4, (int*)S->P.stats + s0, Sz * 4, N * 4, kStatRows, hipMemcpyDeviceToHost, S->stream));
-            if (r->t_out) {
-                const size_t ms = (size_t)S->o.max_saves;
-                SCHK(hipMemcpy2DAsync(r->t_out, N * 8, (double*)S->P.t_out + s0, Sz * 8, N * 8, ms, hipMemcpyDeviceToHost, S->stream));
-                SCHK(hipMemcpy2DAsync(r->u_out, N * 8, (double*)S->P.u_out + s0, Sz * 8, N * 8, ms * n, hipMemcpyDeviceToHost, S->stream));
-                if (r->nsaved)
-                    SCHK(hipMemcpyAsync(r->nsaved, (int*)S->P.nsaved + s0, N * 4, hipMemcpyDeviceToHost, S->stream));
+        // results: as many requests at a time as the staging buffer holds; larger
+        // ones and saved points by copies
+        auto result_bytes = [&](const Request* r) { return ((size_t)r->N * (n * 8 + 4 + kStatRows * 4) + 255) & ~(size_t)255; };
+        for (size_t i = 0; i < fin.size();) {
+            size_t used = 0, first = i;
+            int64_t most = 0;
+            int cnt = 0;
+            for (; i < fin.size() && (result_bytes(fin[i]) > kResultBytes || used + result_bytes(fin[i]) <= kResultBytes); i++) {
+                const Request* r = fin[i];
+                const size_t N = (size_t)r->N, s0 = (size_t)r->slot0;
+                if (result_bytes(r) > kResultBytes) {
+                    if (r->u_final)
+                        SCHK(hipMemcpy2DAsync(r->u_final, N * 8, (double*)S->P.u_final + s0, Sz * 8, N * 8, n, hipMemcpyDeviceToHost, S->stream));
+                    SCHK(hipMemcpyAsync(r->retcode, (int*)S->P.retcode + s0, N * 4, hipMemcpyDeviceToHost, S->stream));
+                    if (r->stats)
+                        SCHK(hipMemcpy2DAsync(r->stats, N * 4, (int*)S->P.stats + s0, Sz * 4, N * 4, kStatRows, hipMemcpyDeviceToHost, S->stream));
+                } else {
+                    double* u = (double*)(S->result_buf + used);
+                    int* rc = (int*)(u + n * N);
+                    S->result_tab[cnt++] = {u, rc, rc + N, r->slot0, r->N};
+                    most = std::max(most, r->N);
+                    used += result_bytes(r);
+                }
+                if (r->t_out) {
+                    const size_t ms = (size_t)S->o.max_saves;
+                    SCHK(hipMemcpy2DAsync(r->t_out, N * 8, (double*)S->P.t_out + s0, Sz * 8, N * 8, ms, hipMemcpyDeviceToHost, S->stream));
+                    SCHK(hipMemcpy2DAsync(r->u_out, N * 8, (double*)S->P.u_out + s0, Sz * 8, N * 8, ms * n, hipMemcpyDeviceToHost, S->stream));
+                    if (r->nsaved)
+                        SCHK(hipMemcpyAsync(r->nsaved, (int*)S->P.nsaved + s0, N * 4, hipMemcpyDeviceToHost, S->stream));
+                }
+            }
+            if (cnt > 0) {
+                hipLaunchKernelGGL(serve_result_kernel, dim3((unsigned)((most + 255) / 256), (unsigned)cnt), dim3(256), 0,
+                                   S->stream, S->P, (const ResultEntry*)S->result_tab, n);
+                SCHK(hipGetLastError());
+            }
+            SCHK(hipStreamSynchronize(S->stream));
+            for (int c = 0; first < i; first++) {
+                const Request* r = fin[first];
+                if (result_bytes(r) > kResultBytes) continue;
+                const ResultEntry& e = S->result_tab[c++];
+                if (r->u_final) memcpy(r->u_final, e.u, (size_t)n * r->N * 8);
+                memcpy(r->retcode, e.rc, (size_t)r->N * 4);
+                if (r->stats) memcpy(r->stats, e.st, (size_t)kStatRows * r->N * 4);
             }
         }
-        if (!fin.empty()) SCHK(hipStreamSynchronize(S->stream));
         if (!fin.empty()) {
             std::lock_guard<std::mutex> lk(S->mu);
             const double t = now_s();
