@@ -89,13 +89,12 @@ struct GJTile {
 };
 
 // Offset (floats) of the matrix-vector result in the Gauss-Jordan LDS buffer
-// of tile R; the buffer holds 51 NP + 16 floats:
+// of tile R; the buffer holds 51 NP floats:
 //   pan [2][NP][16]  the panel, then its multipliers (alternating by panel parity)
 //   wp  [16][NP]     the panel's pivot rows before the panel's update
 //   scl [NP]         row scales
 //   pst int[NP]      step at which each row became a pivot row (-1: not yet)
 //   zbuf [NP]        matrix-vector result
-//   prow [16]        the current step's pivot row (panel wave)
 template <int R>
 __device__ __forceinline__ constexpr int gj_zbuf_off() { return 50 * 16 * R; }
 
@@ -153,7 +152,6 @@ __device__ __forceinline__ void gj_invert(GJTile<R>& G, int n, int* pk, float* g
     float* wp = gjbuf + 32 * NP;
     float* scl = gjbuf + 48 * NP;
     int* pst = (int*)(gjbuf + 49 * NP);
-    float* prowb = gjbuf + 51 * NP;
     for (int i = tid; i < NP; i += blockDim.x) pst[i] = -1;
     // panel 0
 #pragma unroll
@@ -170,11 +168,18 @@ __device__ __forceinline__ void gj_invert(GJTile<R>& G, int n, int* pk, float* g
         float* pan = pan0 + (b & 1) * 16 * NP;
         // ---- the panel's steps, by one wave ----
         if (w == (b & 3)) {
+            // The key of row i for the pivot search is (|entry| bits & keep) | tag:
+            // larger entries win, ties go to the smaller row; keep and tag are 0 for
+            // rows out of the search.  (A NaN wins; the whole inverse is NaN then,
+            // whichever row comes first.)
             float pv[NQ][16];
-            unsigned used = 0;
+            unsigned keep[NQ], tag[NQ];
+            int prec = 0;      // lane kt: pivot row and scale of step kt
+            float drec = 0.0f;
 #pragma unroll
             for (int q = 0; q < NQ; q++) {
                 const int i = l + 64 * q;
+                bool in = false;
                 if (i < NP) {
 #pragma unroll
                     for (int v4 = 0; v4 < 4; v4++) {
@@ -182,59 +187,50 @@ __device__ __forceinline__ void gj_invert(GJTile<R>& G, int n, int* pk, float* g
                         pv[q][4 * v4] = t4.x; pv[q][4 * v4 + 1] = t4.y;
                         pv[q][4 * v4 + 2] = t4.z; pv[q][4 * v4 + 3] = t4.w;
                     }
-                    if (pst[i] >= 0) used |= 1u << q;
+                    in = i < n && pst[i] < 0;
                 } else {
 #pragma unroll
                     for (int cc = 0; cc < 16; cc++) pv[q][cc] = 0.0f;
                 }
+                keep[q] = in ? 0x7fffff80u : 0u;
+                tag[q] = in ? (unsigned)(127 - i) : 0u;
             }
 #pragma unroll
             for (int kt = 0; kt < 16; kt++) {
                 if (kt >= mc) continue;   // uniform
                 unsigned key = 0;
 #pragma unroll
-                for (int q = 0; q < NQ; q++) {
-                    const int i = l + 64 * q;
-                    if (i < n && !((used >> q) & 1u)) key = max(key, gj_key(pv[q][kt], i));
-                }
+                for (int q = 0; q < NQ; q++) key = max(key, (__float_as_uint(pv[q][kt]) & keep[q]) | tag[q]);
                 key = dpp_wave_max_u32(key);
-                const int p = 127 - (int)(key & 127u);
-                // the pivot row through LDS: its lane writes it and every lane
-                // reads it back after a wave barrier (without the barrier the
-                // compiler may order a lane's read before another lane's write)
-#pragma unroll
-                for (int q = 0; q < NQ; q++)
-                    if (l + 64 * q == p) {
-#pragma unroll
-                        for (int v4 = 0; v4 < 4; v4++)
-                            *(float4*)(prowb + 4 * v4) =
-                                make_float4(pv[q][4 * v4], pv[q][4 * v4 + 1], pv[q][4 * v4 + 2], pv[q][4 * v4 + 3]);
-                    }
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                const int p = 127 - (int)(key & 127u), pl = p & 63;
+                // the pivot row into scalar registers (one instruction a column; an
+                // LDS round trip took longer than the rest of the step)
                 float prow[16];
 #pragma unroll
-                for (int v4 = 0; v4 < 4; v4++) {
-                    const float4 t4 = *(const float4*)(prowb + 4 * v4);
-                    prow[4 * v4] = t4.x; prow[4 * v4 + 1] = t4.y; prow[4 * v4 + 2] = t4.z; prow[4 * v4 + 3] = t4.w;
-                }
+                for (int q = 0; q < NQ; q++)
+                    if (NQ == 1 || (p >> 6) == q) {   // uniform
+#pragma unroll
+                        for (int cc = 0; cc < 16; cc++) prow[cc] = wave_bcast(pv[q][cc], pl);
+                    }
                 const float d = __builtin_amdgcn_rcpf(prow[kt]);
+                prec = (l == kt) ? p : prec;
+                drec = (l == kt) ? d : drec;
 #pragma unroll
                 for (int q = 0; q < NQ; q++) {
-                    const int i = l + 64 * q;
-                    const float gq = (i == p) ? 0.0f : pv[q][kt] * d;
+                    const bool is_p = l + 64 * q == p;
+                    const float ng = is_p ? -0.0f : -(pv[q][kt] * d);
 #pragma unroll
                     for (int cc = 0; cc < 16; cc++)
-                        if (cc != kt) pv[q][cc] = fmaf(-gq, prow[cc], pv[q][cc]);
-                    pv[q][kt] = -gq;
-                    if (i == p) used |= 1u << q;
+                        if (cc != kt) pv[q][cc] = fmaf(ng, prow[cc], pv[q][cc]);
+                    pv[q][kt] = ng;
+                    keep[q] = is_p ? 0u : keep[q];
+                    tag[q] = is_p ? 0u : tag[q];
                 }
-                if (l == 0) {
-                    pk[k0 + kt] = p;
-                    scl[p] = d;
-                    pst[p] = k0 + kt;
-                }
+            }
+            if (l < mc) {
+                pk[k0 + l] = prec;
+                scl[prec] = drec;
+                pst[prec] = k0 + l;
             }
 #pragma unroll
             for (int q = 0; q < NQ; q++) {

@@ -14,7 +14,7 @@
 //   pd   double[32]                       parameters (FP64)
 //   fsc  float[nmax + 32]                 FP32 copies of uprev and p (mixed variant)
 //   piv  int[nmax], perm int[nmax]        row positions (scratch of the LU) and the row gather
-//   gjbuf float[51 NP + 16]               Gauss-Jordan panels, pivot rows, scales and
+//   gjbuf float[51 NP]                    Gauss-Jordan panels, pivot rows, scales and
 //                                         mat-vec result (mixed variant; NP = 16 R,
 //                                         R = ceil(nmax/16); layout in odemi_gj.h)
 //   red  double[32] + int[32]             reductions / broadcasts
@@ -60,14 +60,14 @@ struct WGPtrs {
     int ld;
 };
 
-// Gauss-Jordan LDS buffer (floats), NP = 16 R, R = ceil(nmax / 16): 51 NP +
-// 16 for the blocked form (two panels [NP][16], pivot rows [16][NP], scales,
-// pivot steps, mat-vec result, the current pivot row), which covers the
+// Gauss-Jordan LDS buffer (floats), NP = 16 R, R = ceil(nmax / 16): 51 NP
+// for the blocked form (two panels [NP][16], pivot rows [16][NP], scales,
+// pivot steps, mat-vec result), which covers the
 // element-wise form's 6 NP + 2 R NP (column k and k+1 [2][NP], row staging
 // [2][R][NP], scales, result).
 __host__ __device__ inline int wg_gj_floats(int nmax, bool gj) {
     const int r = (nmax + 15) / 16, np16 = 16 * r;
-    return gj ? 51 * np16 + 16 : 0;
+    return gj ? 51 * np16 : 0;
 }
 
 // w_in_lds: W lives in LDS (LU variants); the Gauss-Jordan variant keeps it in registers.

@@ -694,7 +694,7 @@ size_t wg_shmem_bytes(int nmax, bool mixed, bool saves, bool gj) {
     shmem += (size_t)(13 + (saves ? 3 : 0)) * nmax * 8 + 32 * 8;  // vectors + parameters (<= 32)
     shmem += (size_t)(nmax + 32) * 4 + (size_t)nmax * 8;          // fsc + pf, piv + perm
     shmem = (shmem + 15) & ~(size_t)15;
-    if (gj) shmem += (51 * np16 + 16) * 4;                        // Gauss-Jordan buffers + zbuf
+    if (gj) shmem += 51 * np16 * 4;                        // Gauss-Jordan buffers + zbuf
     shmem = (shmem + 15) & ~(size_t)15;
     shmem += 32 * 8 + 32 * 4;
     return shmem;
