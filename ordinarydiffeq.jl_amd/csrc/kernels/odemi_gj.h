@@ -100,24 +100,30 @@ __device__ __forceinline__ constexpr int gj_zbuf_off() { return 50 * 16 * R; }
 
 // T <- W = J - sigma I for the n x n leading block of J (FP32, row stride
 // ODEMI_GJ_LD), identity outside it.  The diagonal shift is formed in FP64 and
-// rounded once.  (Loading the whole tile unconditionally and selecting the
-// padding afterwards measured 4 % slower on uneven chains: short chains then
-// load their full padded tile.)
+// rounded once.  The 16 R x 16 R block is loaded whole, with the padding selected
+// afterwards: loads behind a condition each waited for the one before (60,000 of
+// the 352,000 cycles of an attempt at n = 128).
 template <int R>
 __device__ __forceinline__ void gj_load(GJTile<R>& G, const float* J, int n, double sigma) {
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63, g = l >> 4, c = l & 15;
 #pragma unroll
     for (int m = 0; m < GJTile<R>::MB; m++) {
         const int I = w + 4 * m;
+        if (I >= R) continue;   // uniform; these blocks are never read
+        const float* row = J + (16 * I + 4 * g) * ODEMI_GJ_LD + c;
+#pragma unroll
+        for (int b = 0; b < R; b++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) G.D[m][b][r] = row[r * ODEMI_GJ_LD + 16 * b];
 #pragma unroll
         for (int b = 0; b < R; b++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 const int i = 16 * I + 4 * g + r, j = 16 * b + c;
-                float v = (i == j) ? 1.0f : 0.0f;
-                if (i < n && j < n) {
-                    v = J[i * ODEMI_GJ_LD + j];
-                    if (i == j) v = (float)fma(-1.0, sigma, (double)v);
+                float v = (i < n && j < n) ? G.D[m][b][r] : 0.0f;
+                if (b == I) {   // uniform: a block on the diagonal
+                    const float s = (float)fma(-1.0, sigma, (double)v);
+                    v = (i == j) ? (i < n ? s : 1.0f) : v;
                 }
                 G.D[m][b][r] = v;
             }

@@ -202,40 +202,47 @@ __device__ __forceinline__ void wg_lu_blocked(double* A, int ld, int n, int* tab
         if (w == 0) lu_panel_rows<NQ>(A, ld, n, k0, tab, perm);
         __syncthreads();
         const int mc = min(kLuNB, n - k0), k1 = k0 + mc;
-        for (int J = 16 * w; J < n; J += 16 * NW) {
-            // Row exchanges and U rows: lanes 0-15 take a column of the block each
-            // and bring in the pivot rows, lanes 16-31 the same columns and move the
-            // displaced rows out.
-            const int c = J + c16;
-            if (l < 32 && c < n && (c < k0 || c >= k1)) {
-                const bool out = l >= 16;
-                int from[kLuNB], to[kLuNB];
-                double t[kLuNB];
+        // Row exchanges and U rows of the wave's blocks, two at a time: lanes 0-15
+        // and 16-31 take a column each and bring in the pivot rows, lanes 32-63 the
+        // same columns and move the displaced rows out.
+        {
+            const bool out = l >= 32;
+            const double* T = A + k0 * ld + k0;
+            double L[kLuNB][kLuNB];
+            int from[kLuNB], to[kLuNB];
 #pragma unroll
-                for (int j = 0; j < kLuNB; j++) {   // mc < kLuNB only in the last panel: row n - 1 again
-                    const int top = (k0 + min(j, mc - 1)) * ld;
-                    const int s = tab[min(j, mc - 1)], d = tab[kLuNB + min(j, mc - 1)];
-                    from[j] = out ? top : s;
-                    to[j] = out ? d : top;
-                }
-#pragma unroll
-                for (int j = 0; j < kLuNB; j++) t[j] = A[from[j] + c];
-                if (c >= k1) {   // then mc == kLuNB
-                    const double* T = A + k0 * ld + k0;
-#pragma unroll
-                    for (int j = 1; j < kLuNB; j++) {
-                        double x = t[j];
-#pragma unroll
-                        for (int i = 0; i < j; i++) x = fma(-T[j * ld + i], t[i], x);
-                        t[j] = out ? t[j] : x;
-                    }
-                }
-#pragma unroll
-                for (int j = 0; j < kLuNB; j++)
-                    if (to[j] >= 0) A[to[j] + c] = t[j];
+            for (int j = 0; j < kLuNB; j++) {   // mc < kLuNB only in the last panel: row n - 1 again
+                const int top = (k0 + min(j, mc - 1)) * ld;
+                const int s = tab[min(j, mc - 1)], d = tab[kLuNB + min(j, mc - 1)];
+                from[j] = out ? top : s;
+                to[j] = out ? d : top;
             }
-            lu_wave_sync();
+#pragma unroll
+            for (int j = 1; j < kLuNB; j++)
+#pragma unroll
+                for (int i = 0; i < j; i++) L[j][i] = T[min(j, mc - 1) * ld + i];
+            for (int J = 16 * w; J < n; J += 32 * NW) {
+                const int c = J + c16 + ((l & 16) ? 16 * NW : 0);
+                if (c < n && (c < k0 || c >= k1)) {
+                    double t[kLuNB];
+#pragma unroll
+                    for (int j = 0; j < kLuNB; j++) t[j] = A[from[j] + c];
+                    if (c >= k1 && !out) {   // then mc == kLuNB
+#pragma unroll
+                        for (int j = 1; j < kLuNB; j++)
+#pragma unroll
+                            for (int i = 0; i < j; i++) t[j] = fma(-L[j][i], t[i], t[j]);
+                    }
+#pragma unroll
+                    for (int j = 0; j < kLuNB; j++)
+                        if (to[j] >= 0) A[to[j] + c] = t[j];
+                }
+            }
+        }
+        lu_wave_sync();
+        for (int J = 16 * w; J < n; J += 16 * NW) {
             if (k1 >= n || J + 16 <= k1) continue;   // uniform
+            const int c = J + c16;
             // The block's trailing rows: a 16 x 16 tile's values are loaded while the
             // one above is on the matrix cores.  Only the last tile can be short.
             const int jc = min(c, n - 1);

@@ -355,20 +355,35 @@ __device__ __forceinline__ void wg_save_point(Ctl& c, double& tlast, const Param
     tlast = t;
 }
 
-// sum of v[i]^2 as the index-order fma chain, eight loads ahead of it
+// sum of v[i]^2 as the index-order fma chain, eight loads ahead of it; the last
+// eight are padded with zeros, which leave a sum of squares as it is
 __device__ __forceinline__ double wg_sum_squares(const double* v, int n) {
     double s = 0.0, x[8], y[8];
 #pragma unroll
-    for (int j = 0; j < 8; j++) x[j] = v[min(j, n - 1)];
-    for (int i = 0; i < n; i += 8) {
-#pragma unroll
-        for (int j = 0; j < 8; j++) y[j] = v[min(i + 8 + j, n - 1)];
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            if (i + j < n) s = fma(x[j], x[j], s);
-            x[j] = y[j];
-        }
+    for (int j = 0; j < 8; j++) {
+        const double a = v[min(j, n - 1)];
+        x[j] = (j < n) ? a : 0.0;
     }
+    int i = 0;
+    for (; i + 16 <= n; i += 8) {
+#pragma unroll
+        for (int j = 0; j < 8; j++) y[j] = v[i + 8 + j];
+#pragma unroll
+        for (int j = 0; j < 8; j++) s = fma(x[j], x[j], s);
+#pragma unroll
+        for (int j = 0; j < 8; j++) x[j] = y[j];
+    }
+    int left = n - i - 8;   // 0 .. 7 beyond the eight in x, or n < 8
+    asm("" : "+v"(left));   // selected, not branched around
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        const double a = v[min(i + 8 + j, n - 1)];
+        y[j] = (j < left) ? a : 0.0;
+    }
+#pragma unroll
+    for (int j = 0; j < 8; j++) s = fma(x[j], x[j], s);
+#pragma unroll
+    for (int j = 0; j < 8; j++) s = fma(y[j], y[j], s);
     return s;
 }
 // Index-order fma-chain norms, evaluated by one thread (bit-identical to the
