@@ -317,6 +317,7 @@ struct Tsit5Tab {
                             bt7 = 0.015151515151515152;
 };
 
+typedef const __attribute__((address_space(4))) double* const_f64_ptr;
 __constant__ double kTsitR[7][4] = {
     {1.0, -2.763706197274826, 2.9132554618219126, -1.0530884977290216},
     {0.0, 0.13169999999999998, -0.2234, 0.1017},
@@ -1073,14 +1074,8 @@ __device__ __forceinline__ void tsit5_perform_step(Tsit5Lane<S, K, N>& L, const 
     else L.c.EEst = residual_norm<N>(ea, L.uprev, L.u, P.abstol, P.reltol);
 }
 
-// interpolants.jl:52-64 (@evalpoly Horner via muladd), FP64 evaluation.
 template <typename S, typename K, int N>
-__device__ __forceinline__ void tsit5_interp(const Tsit5Lane<S, K, N>& L, double th, double dt, double* out) {
-    double th2 = th * th;
-    double b[7];
-    b[0] = th * fma(th, fma(th, fma(th, kTsitR[0][3], kTsitR[0][2]), kTsitR[0][1]), kTsitR[0][0]);
-#pragma unroll
-    for (int s = 1; s < 7; s++) b[s] = th2 * fma(th, fma(th, kTsitR[s][3], kTsitR[s][2]), kTsitR[s][1]);
+__device__ __forceinline__ void tsit5_interp_sum(const Tsit5Lane<S, K, N>& L, const double (&b)[7], double dt, double* out) {
 #pragma unroll
     for (int i = 0; i < N; i++) {
         double acc = (double)L.k1[i] * b[0];
@@ -1092,6 +1087,42 @@ __device__ __forceinline__ void tsit5_interp(const Tsit5Lane<S, K, N>& L, double
         acc = fma((double)L.k7[i], b[6], acc);
         out[i] = fma(dt, acc, (double)L.uprev[i]);
     }
+}
+// interpolants.jl:52-64 (@evalpoly Horner via muladd), FP64 evaluation.
+template <typename S, typename K, int N>
+__device__ __forceinline__ void tsit5_interp(const Tsit5Lane<S, K, N>& L, double th, double dt, double* out) {
+    double th2 = th * th;
+    double b[7];
+    b[0] = th * fma(th, fma(th, fma(th, kTsitR[0][3], kTsitR[0][2]), kTsitR[0][1]), kTsitR[0][0]);
+#pragma unroll
+    for (int s = 1; s < 7; s++) b[s] = th2 * fma(th, fma(th, kTsitR[s][3], kTsitR[s][2]), kTsitR[s][1]);
+    tsit5_interp_sum(L, b, dt, out);
+}
+// The same for use in loops: the table is read (scalar loads) where it is used,
+// because the compiler otherwise keeps its 22 values in scalar registers that it
+// does not have and fetches each with two v_readlane an iteration; and fma takes
+// its constant addend from scalar registers (the compiler copies it first).
+__device__ __forceinline__ double fma_vvs(double x, double y, double z) {   // z wave-uniform
+    double r;
+    asm("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "v"(x), "v"(y), "s"(z));
+    return r;
+}
+__device__ __forceinline__ double fma_vsv(double x, double y, double z) {   // y, z wave-uniform
+    double r;
+    asm("v_mov_b64 %0, %1" : "=v"(r) : "s"(z));
+    asm("v_fma_f64 %0, %1, %2, %0" : "+v"(r) : "v"(x), "s"(y));
+    return r;
+}
+template <typename S, typename K, int N>
+__device__ __forceinline__ void tsit5_interp_in_loop(const Tsit5Lane<S, K, N>& L, double th, double dt, double* out) {
+    const_f64_ptr R = (const_f64_ptr)&kTsitR[0][0];
+    asm volatile("" : "+s"(R));
+    double th2 = th * th;
+    double b[7];
+    b[0] = th * fma_vvs(th, fma_vvs(th, fma_vsv(th, R[3], R[2]), R[1]), R[0]);
+#pragma unroll
+    for (int s = 1; s < 7; s++) b[s] = th2 * fma_vvs(th, fma_vsv(th, R[4 * s + 3], R[4 * s + 2]), R[4 * s + 1]);
+    tsit5_interp_sum(L, b, dt, out);
 }
 
 // savevalues! (integrator_utils.jl:340-414); returns savedexactly.
@@ -1212,6 +1243,10 @@ __device__ __forceinline__ void lane_interp(const Tsit5Lane<S, K, N>& L, double 
     tsit5_interp(L, th, L.c.dt, v);
 }
 template <typename S, typename K, int N>
+__device__ __forceinline__ void lane_interp_in_loop(const Tsit5Lane<S, K, N>& L, double th, double* v) {
+    tsit5_interp_in_loop(L, th, L.c.dt, v);
+}
+template <typename S, typename K, int N>
 __device__ __forceinline__ void lane_addsteps(Tsit5Lane<S, K, N>& L, const Params& P) {
     (void)P;
     tsit5_addsteps(L);
@@ -1228,6 +1263,54 @@ __device__ __forceinline__ double ccb_condition(Lane& L, double abst) {
     double v[N];
     lane_interp(L, (abst - c.tprev) / c.dt, v);
     return (double)OdemiCcb<CB>::template cond<double>(v, L.p, abst);
+}
+
+// The states of one step's event search at many times: the division by dt by its
+// refined reciprocal, the IEEE quotient bit for bit while |abst - tprev| is above
+// `tiny` (infinite for a dt out of range); at t and tprev the states there.
+// Bound: vector issue, ~90 instructions a bisection step against 155 with the
+// IEEE quotient, the three cases of the condition apart and the dense output's
+// table in spilled registers: 500,009 bouncing balls, FP64, ~225 conditions
+// each, 1.15 -> 0.77 ms.
+struct StepTheta {
+    double rdt, tiny;
+    __device__ __forceinline__ explicit StepTheta(double dt) {
+        const double a = fabs(dt);
+        rdt = rcp_nr(dt);
+        tiny = (a > 0x1p-400 && a < 0x1p400) ? 0x1p-400 : __builtin_huge_val();
+    }
+};
+template <int N, typename Lane>
+__device__ __forceinline__ void step_state(const Lane& L, const StepTheta& S, double abst, double* v) {
+    const Ctl& c = L.c;
+    const double a = abst - c.tprev;
+    const unsigned long long odd = __ballot(!(fabs(a) > S.tiny) || abst == c.t);
+    double th = div_by_rcp(a, c.dt, S.rdt);
+    if (odd != 0) {   // uniform; the asm keeps the branch from being turned into selects
+        asm volatile("");
+        th = a / c.dt;
+    }
+    lane_interp_in_loop(L, th, v);
+    if (odd != 0) {
+        asm volatile("");
+        const bool at_t = abst == c.t, at_prev = abst == c.tprev;
+#pragma unroll
+        for (int i = 0; i < N; i++) v[i] = at_t ? (double)L.u[i] : at_prev ? (double)L.uprev[i] : v[i];
+    }
+}
+template <int CB, int N, typename Lane>
+__device__ __forceinline__ double ccb_condition_dense(Lane& L, const StepTheta& S, double abst) {
+    double v[N];
+    L.c.ncond++;
+    step_state<N>(L, S, abst, v);
+    return (double)OdemiCcb<CB>::template cond<double>(v, L.p, abst);
+}
+template <int CB, int N, typename Lane>
+__device__ __forceinline__ void vcb_condition_dense(Lane& L, const StepTheta& S, double abst, double* out) {
+    double v[N];
+    L.c.ncond++;
+    step_state<N>(L, S, abst, v);
+    OdemiCcb<CB>::template vcond<double>(out, v, L.p, abst);
 }
 
 // is_event_occurrence (callbacks.jl:525-530)
@@ -1256,6 +1339,7 @@ __device__ bool ccb_find_time(Lane& L, double& cb_t, double& bottom_sign, double
         bc = ccb_condition<CB, N>(L, bottom_t);
     }
     const double bs = jl_sign(bc);
+    const StepTheta S(c.dt);
     double top_t = c.t;
     double ts = jl_sign(ccb_condition<CB, N>(L, top_t));
     bool ev = ccb_is_event<CB>(bs, ts);
@@ -1263,7 +1347,7 @@ __device__ bool ccb_find_time(Lane& L, double& cb_t, double& bottom_sign, double
         const double h = (c.t - c.tprev) / (double)(C::interp_points - 1);
         for (int i = 2; i <= C::interp_points; i++) {
             top_t = (i == C::interp_points) ? c.t : fma((double)(i - 1), h, c.tprev);
-            ts = jl_sign(ccb_condition<CB, N>(L, top_t));
+            ts = jl_sign(ccb_condition_dense<CB, N>(L, S, top_t));
             ev = ccb_is_event<CB>(bs, ts);
             if (ev) break;
         }
@@ -1275,10 +1359,10 @@ __device__ bool ccb_find_time(Lane& L, double& cb_t, double& bottom_sign, double
     for (int it = 0; it < 2200; it++) {
         const double m = l + 0.5 * (r - l);
         if (m == l || m == r) break;
-        const double sm = jl_sign(ccb_condition<CB, N>(L, m));
-        if (sm == 0.0) { l = m; r = m; break; }
-        if (sm == bs) l = m;
-        else r = m;
+        // bs is 1 or -1; a zero closes the bracket on m
+        const double w = bs * ccb_condition_dense<CB, N>(L, S, m);
+        l = (w >= 0.0) ? m : l;
+        r = (w > 0.0) ? r : m;
     }
     cb_t = (C::rootfind == 1) ? r : l;
     residual = ccb_condition<CB, N>(L, cb_t);
@@ -1387,6 +1471,7 @@ __device__ bool vcb_find_time(Lane& L, double& cb_t, double* ev, double& residua
         for (int i = 0; i < V; i++)
             if ((prev >> i) & 1u) bs[i] = jl_sign(tmp[i]);
     }
+    const StepTheta S(c.dt);
     double top_t = c.t;
     vcb_condition<CB, N>(L, top_t, top);
     unsigned mask = vcb_events<V>(bs, top);
@@ -1395,7 +1480,7 @@ __device__ bool vcb_find_time(Lane& L, double& cb_t, double* ev, double& residua
         const double h = (c.t - c.tprev) / (double)(C::interp_points - 1);
         for (int i = 2; i <= C::interp_points; i++) {
             top_t = (i == C::interp_points) ? c.t : fma((double)(i - 1), h, c.tprev);
-            vcb_condition<CB, N>(L, top_t, top);
+            vcb_condition_dense<CB, N>(L, S, top_t, top);
             mask = vcb_events<V>(bs, top);
             if (mask) break;
         }
@@ -1423,7 +1508,7 @@ __device__ bool vcb_find_time(Lane& L, double& cb_t, double* ev, double& residua
             for (int it = 0; it < 2200; it++) {
                 const double m = l + 0.5 * (r - l);
                 if (m == l || m == r) break;
-                vcb_condition<CB, N>(L, m, tmp);
+                vcb_condition_dense<CB, N>(L, S, m, tmp);
                 const double sm = jl_sign(tmp[idx]);
                 if (sm == 0.0) { l = m; r = m; break; }
                 if (sm == bs[idx]) l = m;
@@ -2332,6 +2417,10 @@ __device__ __forceinline__ void lane_interp(const RodasLane<F, N>& L, double th,
     rodas_interp(L, th, v);
 }
 template <typename F, int N>
+__device__ __forceinline__ void lane_interp_in_loop(const RodasLane<F, N>& L, double th, double* v) {
+    rodas_interp(L, th, v);
+}
+template <typename F, int N>
 __device__ __forceinline__ void lane_addsteps(RodasLane<F, N>& L, const Params& P) {
     rodas_addsteps(L, P);
 }
@@ -2405,7 +2494,6 @@ __device__ __forceinline__ int rodas_attempt(RodasLane<F, N>& L, const Params& P
 // stage sums of the last stages that share their first five terms, and the
 // controller's rules.
 // ---------------------------------------------------------------------------
-typedef const __attribute__((address_space(4))) double* const_f64_ptr;
 
 // Dense LU on registers: the arithmetic of lu_factor_reg / lu_solve_reg.
 template <typename T, int N>
