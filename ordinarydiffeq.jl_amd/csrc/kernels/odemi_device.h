@@ -886,6 +886,13 @@ __device__ __forceinline__ void tsit5_init(Tsit5Lane<S, K, N>& L, const Params& 
     }
     L.c.dtpropose = L.c.dt;
 }
+// What the prep kernels clear for the persistent kernel behind them: the work
+// queue's counters and the trajectory's saved-point count (fills of their own
+// cost a small solve two launches).
+__device__ __forceinline__ void prep_clear(const Params& P, i64 j) {
+    if (j < 8) P.counters[j] = 0;
+    if (P.nsaved && j < P.N) P.nsaved[j] = 0;
+}
 // One thread per trajectory, ahead of the persistent kernel: the start-up work
 // (one RHS in the stage precision, initdt's two FP64 RHS and norms) runs fully
 // parallel instead of stalling the other lanes of a wave whenever one lane
@@ -893,6 +900,7 @@ __device__ __forceinline__ void tsit5_init(Tsit5Lane<S, K, N>& L, const Params& 
 template <typename S, typename K, int N>
 __device__ void tsit5_prep(const Params& P) {
     const i64 j = (i64)blockIdx.x * blockDim.x + threadIdx.x;
+    prep_clear(P, j);
     if (j >= P.N) return;
     Tsit5Lane<S, K, N> L;
     double u0d[N], pd[ODEMI_NP];
@@ -2164,6 +2172,7 @@ __device__ __forceinline__ void rodas_init(RodasLane<F, N>& L, const Params& P, 
 template <int N>
 __device__ void rodas_prep(const Params& P) {
     const i64 j = (i64)blockIdx.x * blockDim.x + threadIdx.x;
+    prep_clear(P, j);
     if (j >= P.N) return;
     Ctl c;
     ctl_init(c, P, j);

@@ -785,12 +785,21 @@ int solve_impl(odemi_ctx* ctx, odemi_rhs* rhs, odemi_solve_args* a, bool noalloc
         if (!plain) fn_prep = rhs->rodas_prep;
     }
     if (plain && mixed) { ctx->err = "the plain engine is FP64 only"; return -3; }
+    // Longest first only where the order matters.  Up to one workgroup of 256
+    // lanes per CU every lane takes one trajectory and every wave has its SIMD to
+    // itself: the solve lasts as long as its longest trajectory in any order, and
+    // the sort's three kernels, its fill and the records' unpacking are launches
+    // saved (1,024 Lorenz trajectories 277 -> 256 us a call; at 65,536 the longest
+    // wave is the same, above it waves share a SIMD and short ones should leave
+    // together).
+    const bool sorted = a->sort_by_cost && !plain && N > 0 &&
+                        ((rodas && (rhs->flags & ODEMI_COMPILE_WG)) || N > 256 * (int64_t)std::max(ctx->cu_count, 1));
     // queue-order records (final-state-only Tsit5 persistent engine, no save
     // before the end point, no lane callbacks; not in the allocation-free form;
     // $ODEMI_QUEUE_RECORDS=0 reads and writes the SoA arrays in place instead)
     const char* qr = getenv("ODEMI_QUEUE_RECORDS");
     const bool use_rec = !(qr && atoi(qr) == 0) && !rodas && !plain && !noalloc && fn_prep && rhs->rec_unpack &&
-                         a->sort_by_cost && N > 0 &&
+                         sorted &&
                          a->nsaveat == 0 && !a->save_everystep && !a->save_start && !(rhs->features & 6) &&
                          nmax == rhs->n;
     const int rec_np = std::max(rhs->np, 1);
@@ -854,7 +863,7 @@ int solve_impl(odemi_ctx* ctx, odemi_rhs* rhs, odemi_solve_args* a, bool noalloc
     size_t need = 0;
     auto add = [&](size_t b) { need += ((b + 255) & ~size_t(255)); };
     add(64);                                   // counters
-    if (a->sort_by_cost && !plain) {
+    if (sorted) {
         if (N > 0x7fffffffLL) { ctx->err = "N too large for the work-queue order"; return -2; }
         add(N_ * 4); add(kCostBins * 4);
     }
@@ -894,7 +903,7 @@ int solve_impl(odemi_ctx* ctx, odemi_rhs* rhs, odemi_solve_args* a, bool noalloc
     P.save_end_user = a->save_end_user; P.max_saves = a->max_saves;
     P.refine_sweeps = a->refine_sweeps;
     P.counters = (unsigned long long*)ar.take(64);
-    if (clear_words(ctx, P.counters, 16, s, noalloc)) return -1;
+    if (!fn_prep && clear_words(ctx, P.counters, 16, s, noalloc)) return -1;   // else by the prep kernel
     if (dev) {
         P.u0 = a->u0; P.p = a->p; P.t0 = a->t0; P.tf = a->tf; P.saveat = a->saveat; P.nvec = a->nvec;
         P.tstops = a->tstops;
@@ -927,7 +936,7 @@ int solve_impl(odemi_ctx* ctx, odemi_rhs* rhs, odemi_solve_args* a, bool noalloc
             P.nvec = nv;
         }
     }
-    if (a->sort_by_cost && !plain && N > 0) {
+    if (sorted) {
         int* ord = (int*)ar.take(N_ * 4);
         unsigned* bins = (unsigned*)ar.take(kCostBins * 4);
         const int g = (int)((N + kCostTile - 1) / kCostTile);
@@ -978,7 +987,7 @@ int solve_impl(odemi_ctx* ctx, odemi_rhs* rhs, odemi_solve_args* a, bool noalloc
         P.pre_dt = (double*)ar.take(N_ * 8);
         if (!rodas) P.pre_k1 = (double*)ar.take(N_ * nmax * 8);
     }
-    if (P.nsaved && clear_words(ctx, P.nsaved, N_, s, noalloc)) return -1;
+    if (!fn_prep && P.nsaved && clear_words(ctx, P.nsaved, N_, s, noalloc)) return -1;
 
     int64_t launches = 0;
     // kernel_ms: the plain engine's launches, or the persistent kernel alone

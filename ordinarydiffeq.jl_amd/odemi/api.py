@@ -559,8 +559,8 @@ def solve_arrays(fun, alg, u0, p, t0, tf, ensemblealg=None, *, reltol=None, abst
         u0c = u0.contiguous()
         pc = (p.contiguous() if p is not None else torch.zeros((1, N), **dd))
         t0c, tfc = t0.contiguous(), tf.contiguous()
-        sat = torch.as_tensor(sa, **dd) if len(sa) else torch.zeros(1, **dd)
-        tst = torch.as_tensor(tsv, **dd) if len(tsv) else torch.zeros(1, **dd)
+        sat = torch.as_tensor(sa, **dd) if len(sa) else torch.empty(1, **dd)
+        tst = torch.as_tensor(tsv, **dd) if len(tsv) else torch.empty(1, **dd)
         out = outputs or {}
         o = dict(
             t_out=out.get("t_out", torch.empty((max(max_saves, 1), N), **dd)),
