@@ -1082,11 +1082,21 @@ int solve_impl(odemi_ctx* ctx, odemi_rhs* rhs, odemi_solve_args* a, bool noalloc
         launches++;
     }
     if (!dev) {
-        if (ms_ > 0) {
-            HIPCHK(ctx, hipMemcpyAsync(a->t_out, P.t_out, N_ * ms_ * 8, hipMemcpyDeviceToHost, s));
-            HIPCHK(ctx, hipMemcpyAsync(a->u_out, P.u_out, N_ * ms_ * nmax * 8, hipMemcpyDeviceToHost, s));
-        }
         if (a->nsaved) HIPCHK(ctx, hipMemcpyAsync(a->nsaved, P.nsaved, N_ * 4, hipMemcpyDeviceToHost, s));
+        if (ms_ > 0) {
+            // Where every step may be saved the capacity is a guess (4,096 points by
+            // default: 65 MB for 500 Lorenz trajectories that use 50 of them): only
+            // rows that some trajectory reached hold values and are copied.
+            size_t rows = ms_;
+            if (a->nsaved && ms_ > (size_t)a->nsaveat + 2) {
+                HIPCHK(ctx, hipStreamSynchronize(s));
+                rows = std::min(ms_, (size_t)std::max(*std::max_element(a->nsaved, a->nsaved + N), 0));
+            }
+            if (rows > 0) {
+                HIPCHK(ctx, hipMemcpyAsync(a->t_out, P.t_out, N_ * rows * 8, hipMemcpyDeviceToHost, s));
+                HIPCHK(ctx, hipMemcpyAsync(a->u_out, P.u_out, N_ * rows * nmax * 8, hipMemcpyDeviceToHost, s));
+            }
+        }
         if (a->u_final) HIPCHK(ctx, hipMemcpyAsync(a->u_final, P.u_final, N_ * nmax * 8, hipMemcpyDeviceToHost, s));
         if (a->t_final) HIPCHK(ctx, hipMemcpyAsync(a->t_final, P.t_final, N_ * 8, hipMemcpyDeviceToHost, s));
         HIPCHK(ctx, hipMemcpyAsync(a->retcode, P.retcode, N_ * 4, hipMemcpyDeviceToHost, s));

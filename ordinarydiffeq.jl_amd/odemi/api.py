@@ -158,11 +158,25 @@ def _autotune(ctx, h, a, key, wg):
     return best
 
 
+class _Seed(list):
+    """The seed of a context's generator that nothing has asked for yet."""
+
+
 class EnsembleContext:
     """Per-trajectory context handed to prob_func/output_func (v7 API)."""
 
     def __init__(self, sim_id, repeat, rng):
-        self.sim_id, self.repeat, self.rng = sim_id, repeat, rng
+        self.sim_id, self.repeat, self._rng = sim_id, repeat, rng
+
+    @property
+    def rng(self):
+        if isinstance(self._rng, _Seed):   # made on first use: ~8 us a trajectory
+            self._rng = np.random.default_rng(list(self._rng))
+        return self._rng
+
+    @rng.setter
+    def rng(self, rng):
+        self._rng = rng
 
     @property
     def i(self):
@@ -684,8 +698,11 @@ def solve(prob, alg, ensemblealg=None, *, trajectories=1, reltol=None, abstol=No
     if max_saves is None and (sev or forced):
         max_saves = 4096
 
+    if N > 0:
+        np.random.default_rng([int(seed), 1])   # refuses a bad seed here, not at its first use
+
     def draw(i, repeat):
-        rng = np.random.default_rng([int(seed), i + 1] if repeat == 1 else [int(seed), i + 1, repeat])
+        rng = _Seed([int(seed), i + 1] if repeat == 1 else [int(seed), i + 1, repeat])
         pi = ens.prob_func(remake(base) if ens.safetycopy else base, EnsembleContext(i + 1, repeat, rng))
         if len(pi.u0) != n or len(pi.p) != np_:
             raise ValueError("all trajectories must share the state and parameter dimensions")
@@ -718,12 +735,16 @@ def solve(prob, alg, ensemblealg=None, *, trajectories=1, reltol=None, abstol=No
         if (sev or forced) and int(o["nsaved"].max(initial=0)) > o["max_saves"]:
             raise RuntimeError(f"the saves (save_everystep / callback save_positions) exceeded max_saves="
                                f"{o['max_saves']} points; pass a larger max_saves")
-        sols = []
-        for j in range(Nb):
-            ns = min(int(o["nsaved"][j]), o["max_saves"])
-            st = o["stats"][:, j]
-            sols.append(ODESolution(o["t_out"][:ns, j].copy(), [o["u_out"][k, :, j].copy() for k in range(ns)],
-                                    ReturnCode(int(o["retcode"][j])), DEStats(*st), probs[j], alg))
+        # trajectory-major copies of the rows in use, then one block per solution,
+        # whose rows are its u: one copy a trajectory instead of one a saved step
+        cap = o["max_saves"]
+        nsaved = [min(k, cap) for k in o["nsaved"].tolist()]
+        rows = max(nsaved, default=0)
+        ts = np.ascontiguousarray(o["t_out"][:rows].T)
+        us = np.ascontiguousarray(o["u_out"][:rows].transpose(2, 0, 1))
+        stats, codes = o["stats"].T.tolist(), o["retcode"].tolist()
+        sols = [ODESolution(ts[j, :ns].copy(), list(us[j, :ns].copy()), ReturnCode(codes[j]), DEStats(*stats[j]),
+                            probs[j], alg) for j, ns in enumerate(nsaved)]
         return sols, o
 
     u_acc = ens.u_init
