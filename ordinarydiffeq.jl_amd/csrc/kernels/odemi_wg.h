@@ -36,6 +36,13 @@
 #ifndef ODEMI_WG_THREADS
 #define ODEMI_WG_THREADS 256
 #endif
+// The FP64 kernels from n = 96 on, whose W leaves room for one workgroup a CU:
+// eight waves, so that two a SIMD cover each other's latency in the trailing
+// updates of the LU (96 chains of n = 8..128: 10.5 -> 10.0 ms; below, eight waves
+// of ~205 registers would halve the workgroups of a CU).
+#ifndef ODEMI_WG_THREADS_F64
+#define ODEMI_WG_THREADS_F64 (ODEMI_N >= 96 ? 512 : ODEMI_WG_THREADS)
+#endif
 #define ODEMI_WG_ROWS ((ODEMI_N + 63) / 64)
 
 #include "odemi_gj.h"

@@ -448,7 +448,8 @@ static std::string build_source(const char* problem_src, int n, int np, int flag
         const char* ww = getenv("ODEMI_WG_MIN_WAVES");
         const int wgw = (ww && *ww) ? atoi(ww) : 3;
         for (auto& k : v) {
-            s << "extern \"C\" __global__ void __launch_bounds__(ODEMI_WG_THREADS) ";
+            s << "extern \"C\" __global__ void __launch_bounds__("
+              << (k[1][0] == 'f' ? "ODEMI_WG_THREADS" : "ODEMI_WG_THREADS_F64") << ") ";
             if (wgw > 0 && k[1][0] == 'f') s << "__attribute__((amdgpu_waves_per_eu(" << wgw << "))) ";
             s << k[0] << "(odemi::Params P) { odemi::rodas_wg_impl<" << k[1] << ", " << k[2] << ", " << k[3]
               << ">(P); }\n";
@@ -458,7 +459,8 @@ static std::string build_source(const char* problem_src, int n, int np, int flag
                                 {"odemi_rodas_wg_serve_init_mixed", "rodas_wg_serve_init", "float", "(ODEMI_GJ != 0)"},
                                 {"odemi_rodas_wg_serve_tick_mixed", "rodas_wg_serve_tick", "float", "(ODEMI_GJ != 0)"}};
         for (auto& k : sv) {
-            s << "extern \"C\" __global__ void __launch_bounds__(ODEMI_WG_THREADS) ";
+            s << "extern \"C\" __global__ void __launch_bounds__("
+              << (k[2][0] == 'f' ? "ODEMI_WG_THREADS" : "ODEMI_WG_THREADS_F64") << ") ";
             if (wgw > 0 && k[2][0] == 'f') s << "__attribute__((amdgpu_waves_per_eu(" << wgw << "))) ";
             s << k[0] << "(odemi::Params P) { odemi::" << k[1] << "<" << k[2] << ", " << k[3] << ">(P); }\n";
         }
@@ -682,6 +684,10 @@ int ensure_ws(odemi_ctx* c, size_t bytes) {
     return 0;
 }
 
+// Threads of the workgroup kernels: ODEMI_WG_THREADS, for the FP64 variant
+// ODEMI_WG_THREADS_F64 (kernels/odemi_wg.h).
+int wg_threads(int nmax, bool mixed) { return !mixed && nmax >= 96 ? 512 : 256; }
+
 // Row stride (and side) of each workgroup's FP32 Jacobian block in the mixed
 // workgroup kernels: 16 ceil(nmax / 16), as ODEMI_GJ_LD in kernels/odemi_gj.h.
 size_t gj_ld(int nmax) { return 16 * (((size_t)nmax + 15) / 16); }
@@ -826,7 +832,7 @@ int solve_impl(odemi_ctx* ctx, odemi_rhs* rhs, odemi_solve_args* a, bool noalloc
     const size_t vrows = plain_wg ? 3 : rodas ? (size_t)(3 + nmax) : 4;
     // ---- launch geometry of the persistent kernels ----
     const int block = a->block > 0 ? a->block : 256;
-    const int threads = use_wg ? 256 : block;   // ODEMI_WG_THREADS for the workgroup kernels
+    const int threads = use_wg ? wg_threads(nmax, mixed) : block;
     const bool use_gj = use_wg && mixed && nmax <= 128;   // register-tiled Gauss-Jordan variant
     size_t shmem = 0;
     int64_t grid = 0;
@@ -856,7 +862,7 @@ int solve_impl(odemi_ctx* ctx, odemi_rhs* rhs, odemi_solve_args* a, bool noalloc
         shmem = wg_shmem_bytes(nmax, false, (rhs->features & 16) != 0, false);
         if (shmem > 160 * 1024) { ctx->err = "state dimension too large for the workgroup kernel's LDS"; return -3; }
         int nb = 0;
-        HIPCHK(ctx, hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn_main, 256, shmem));
+        HIPCHK(ctx, hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn_main, wg_threads(nmax, false), shmem));
         grid = std::min<int64_t>((int64_t)std::max(nb, 1) * std::max(ctx->cu_count, 1), N);
     }
     // ---- workspace layout ----
@@ -1002,7 +1008,7 @@ int solve_impl(odemi_ctx* ctx, odemi_rhs* rhs, odemi_solve_args* a, bool noalloc
         const int lgrid = (int)((N + block - 1) / block);
         if (plain_wg) {
             // init: one workgroup per trajectory (grid-strided)
-            if (launch(ctx, fn_init, (int)grid, 256, P, s, shmem)) return -1;
+            if (launch(ctx, fn_init, (int)grid, wg_threads(nmax, false), P, s, shmem)) return -1;
         } else {
             if (launch(ctx, fn_init, lgrid, block, P, s)) return -1;
         }
@@ -1015,7 +1021,7 @@ int solve_impl(odemi_ctx* ctx, odemi_rhs* rhs, odemi_solve_args* a, bool noalloc
             for (int k = 0; k < kBatch; k++) {
                 if (plain_wg) {
                     if (clear_words(ctx, P.counters, 2, s, true)) return -1;
-                    if (launch(ctx, fn_main, (int)grid, 256, P, s, shmem)) return -1;
+                    if (launch(ctx, fn_main, (int)grid, wg_threads(nmax, false), P, s, shmem)) return -1;
                 } else {
                     if (k == kBatch - 1 && clear_words(ctx, P.counters + 1, 2, s, true)) return -1;
                     if (launch(ctx, fn_main, lgrid, block, P, s)) return -1;
@@ -1352,7 +1358,7 @@ extern "C" odemi_server* odemi_server_create(odemi_ctx* ctx, odemi_rhs* rhs, con
         S->shmem = wg_shmem_bytes(n, pi == 1, (rhs->features & 16) != 0, S->gj);   // dense rows for events
         if (S->shmem > 160 * 1024) { ctx->err = "state dimension too large for the workgroup kernel's LDS"; delete S; return nullptr; }
         int nb = 0;
-        if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&nb, rhs->wg_serve_tick[pi], 256, S->shmem) != hipSuccess)
+        if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&nb, rhs->wg_serve_tick[pi], wg_threads(n, pi == 1), S->shmem) != hipSuccess)
             nb = 1;
         S->wg_grid = std::max(nb, 1) * std::max(ctx->cu_count, 1);
     }
@@ -1657,6 +1663,7 @@ static void server_loop(odemi_server* S) {
                                  : (S->o.max_saves > 0 ? S->rhs->serve_tick_sv[S->o.alg][pi]
                                                        : S->rhs->serve_tick[S->o.alg][pi]);
     const size_t Sz = (size_t)S->S;
+    const unsigned wg_block = (unsigned)wg_threads(n, pi == 1);
     for (;;) {
         std::vector<Request*> admit;
         int64_t high = 0;
@@ -1734,7 +1741,7 @@ static void server_loop(odemi_server* S) {
             Pi.nslots = N;
             void* args[] = {&Pi};
             if (S->wg)   // one workgroup per admitted slot
-                SCHK(hipModuleLaunchKernel(f_init, (unsigned)std::min<int64_t>(N, S->wg_grid), 1, 1, 256, 1, 1,
+                SCHK(hipModuleLaunchKernel(f_init, (unsigned)std::min<int64_t>(N, S->wg_grid), 1, 1, wg_block, 1, 1,
                                            (unsigned)S->shmem, S->stream, args, nullptr));
             else
                 SCHK(hipModuleLaunchKernel(f_init, (unsigned)((N + 255) / 256), 1, 1, 256, 1, 1, 0, S->stream, args, nullptr));
@@ -1746,7 +1753,7 @@ static void server_loop(odemi_server* S) {
             Pt.slot0 = 0;
             Pt.nslots = high;
             void* args[] = {&Pt};
-            SCHK(hipModuleLaunchKernel(f_tick, (unsigned)std::min<int64_t>(high, S->wg_grid), 1, 1, 256, 1, 1,
+            SCHK(hipModuleLaunchKernel(f_tick, (unsigned)std::min<int64_t>(high, S->wg_grid), 1, 1, wg_block, 1, 1,
                                        (unsigned)S->shmem, S->stream, args, nullptr));
         } else if (high > 0) {
             Params Pt = S->P;

@@ -11,12 +11,12 @@ from odemi import problems as P
 
 pytestmark = pytest.mark.gpu
 
-EDGES = (2, 6, 8, 10, 14, 16, 18, 24, 30, 32, 34, 62, 64, 66, 70, 72, 74)
+EDGES = (2, 6, 8, 10, 14, 16, 18, 24, 30, 32, 34, 62, 64, 66, 70, 72, 74, 96, 98, 112, 126, 128)
 
 
 # scale 1e-130: dividends below the range of the short quotient, so every
 # substitution goes through the IEEE divisions (alpha = 0: a linear chain)
-@pytest.mark.parametrize("nmax,scale", [(10, 1.0), (18, 1.0), (66, 1.0), (74, 1.0), (18, 1e-130)])
+@pytest.mark.parametrize("nmax,scale", [(10, 1.0), (18, 1.0), (66, 1.0), (74, 1.0), (128, 1.0), (18, 1e-130)])
 def test_lu_edges_bit_identical(nmax, scale):
     sizes = [n for n in EDGES if n <= nmax]
     d = P.chain_ensemble(N=4 * len(sizes), seed=31, m_lo=nmax // 2, m_hi=nmax // 2)
