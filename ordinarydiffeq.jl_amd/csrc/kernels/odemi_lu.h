@@ -9,8 +9,8 @@
 //
 // Bound: the instruction latency of one wave (a chain of 2 n substitution steps
 // a solve, n pivot steps a factorization), one trajectory a workgroup.  Measured
-// alone on a CU at n = 128: factorization 76 us (81,000 of 182,000 cycles in the
-// panels), solve 8 us; 96 chains of n = 8..128 together 43.9 -> 11.3 ms against
+// alone on a CU at n = 128: factorization ~60 us (85,000 cycles of it in the
+// panels), solve 8 us; 96 chains of n = 8..128 together 43.2 -> 10.0 ms against
 // the element-by-element factorization and IEEE quotients in every step.
 #pragma once
 
