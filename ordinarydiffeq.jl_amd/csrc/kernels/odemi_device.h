@@ -3002,8 +3002,10 @@ __device__ void tsit5_serve_tick(const Params& P0) {
     if constexpr (kFastAttempts) {
         fast_to_ctl(F, L.c, P);
         fast_counts(F, L.c);
+        if (L.c.accept_step) {   // a rejected trial state stays: a trajectory that fails next reports it
 #pragma unroll
-        for (int i = 0; i < N; i++) { L.u[i] = L.uprev[i]; L.k7[i] = L.k1[i]; }
+            for (int i = 0; i < N; i++) { L.u[i] = L.uprev[i]; L.k7[i] = L.k1[i]; }
+        }
     }
     plain_store_ctl<N>(L.c, P, j, 1);
     tsit5_store_state(L, P, j);
