@@ -33,15 +33,18 @@
 #pragma once
 #ifdef ODEMI_WITH_WG
 
-#ifndef ODEMI_WG_THREADS
+// Threads of a workgroup (the host reads them back from the module): 256.
 #define ODEMI_WG_THREADS 256
-#endif
 // The FP64 kernels from n = 96 on, whose W leaves room for one workgroup a CU:
 // eight waves, so that two a SIMD cover each other's latency in the trailing
 // updates of the LU (96 chains of n = 8..128: 10.5 -> 10.0 ms; below, eight waves
-// of ~205 registers would halve the workgroups of a CU).
-#ifndef ODEMI_WG_THREADS_F64
-#define ODEMI_WG_THREADS_F64 (ODEMI_N >= 96 ? 512 : ODEMI_WG_THREADS)
+// of ~205 registers would halve the workgroups of a CU).  Four with continuous
+// callbacks, whose kernels take up to 256 registers and 8 accumulation registers:
+// a CU does not hold eight waves of those, and such a launch is refused.
+#if ODEMI_N >= 96 && !defined(ODEMI_NCCB_WG)
+#define ODEMI_WG_THREADS_F64 512
+#else
+#define ODEMI_WG_THREADS_F64 ODEMI_WG_THREADS
 #endif
 #define ODEMI_WG_ROWS ((ODEMI_N + 63) / 64)
 
@@ -303,7 +306,7 @@ __device__ __forceinline__ void wg_negate(double* x, int n) {
 // FP64 residual r = b - J x + sigma x (J x from the traced Jacobian-vector
 // product at uprev).  Scratch: rb (copy of b), r, d -- three free vectors.
 template <typename F>
-__device__ void wg_wsolve(const WGPtrs& S, int n, double* x, double* rb, double* r, double* d,
+__device__ __forceinline__ void wg_wsolve(const WGPtrs& S, int n, double* x, double* rb, double* r, double* d,
                           const double* uprev, const double* p, double t, double sigma, int sweeps) {
     const F* A = (const F*)S.W;
     if constexpr (sizeof(F) == sizeof(double)) {
@@ -761,8 +764,12 @@ __device__ bool wg_vcb_find_time(const WGPtrs& S, Ctl& c, int n, int nmax, doubl
 // and sums round separately except linsolve_tmp = fsalfirst + dtgamma dT;
 // dtC = C ./ dt; the dense rows from the new stages.  The dense rows serve as
 // solve scratch until they are rebuilt.  No stats change.
+// Inlined, as wg_wsolve is: around a call the kernel kept S in memory (flat
+// instead of LDS accesses everywhere) and at n > 64 some 70 values in other
+// registers, and the compiler put copies of those where the exec mask is empty,
+// so that they were lost (tests/test_wg_kernel_code.py looks for such copies).
 template <typename F, bool GJ, int R, typename GT>
-__device__ void wg_addsteps(const WGPtrs& S, const Params& P, const Ctl& c, int n, GT& G, float* Jg) {
+__device__ __forceinline__ void wg_addsteps(const WGPtrs& S, const Params& P, const Ctl& c, int n, GT& G, float* Jg) {
     const int tid = threadIdx.x, NT = blockDim.x;
     const int nmax = P.nmax, ld = S.ld;
     const double t = c.tprev, dt = c.dt;

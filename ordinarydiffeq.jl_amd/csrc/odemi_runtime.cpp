@@ -263,6 +263,7 @@ struct odemi_rhs {
     odemi_ctx* ctx = nullptr;
     hipModule_t mod = nullptr;
     int n = 0, np = 0, flags = 0;
+    int wg_threads[2] = {256, 256};   // of the workgroup kernels [fp64, mixed]
     int features = 0;   // lane hooks 1 isoutofdomain, 2 discrete, 4 continuous callbacks; workgroup callbacks 8, 16
     hipFunction_t tsit5_persist_f64 = nullptr, tsit5_persist_mixed = nullptr;
     hipFunction_t tsit5_persist_f64_sv = nullptr, tsit5_persist_mixed_sv = nullptr;
@@ -438,6 +439,7 @@ static std::string build_source(const char* problem_src, int n, int np, int flag
              " { odemi::rodas_plain_step<ODEMI_N>(P); }\n";
     }
     if (flags & ODEMI_COMPILE_WG) {
+        s << "extern \"C\" __device__ const int odemi_wg_threads[2] = {ODEMI_WG_THREADS_F64, ODEMI_WG_THREADS};\n";
         // the mixed variant uses the register-tiled Gauss-Jordan solver when n <= 128
         const char* v[4][4] = {{"odemi_rodas_wg_f64", "double", "false", "false"},
                                {"odemi_rodas_wg_f64_sv", "double", "true", "false"},
@@ -648,6 +650,24 @@ extern "C" odemi_rhs* odemi_compile_rhs(odemi_ctx* ctx, const char* problem_src,
         get("odemi_rodas_wg_serve_init_mixed", &r->wg_serve_init[1]);
         get("odemi_rodas_wg_serve_tick_f64", &r->wg_serve_tick[0]);
         get("odemi_rodas_wg_serve_tick_mixed", &r->wg_serve_tick[1]);
+        hipDeviceptr_t gp = nullptr;
+        size_t gsz = 0;
+        if (hipModuleGetGlobal(&gp, &gsz, r->mod, "odemi_wg_threads") != hipSuccess || gsz != sizeof(r->wg_threads) ||
+            hipMemcpyDtoH(r->wg_threads, gp, sizeof(r->wg_threads)) != hipSuccess) {
+            ctx->err = "module lacks the odemi_wg_threads words";
+            (void)hipModuleUnload(r->mod);
+            delete r;
+            return nullptr;
+        }
+        // The launch bounds cap a kernel's own registers, not those of the functions
+        // that it calls (a problem whose traced code is not inlined): where a CU
+        // cannot hold the workgroup, four waves, which always fit.
+        const hipFunction_t f64[] = {r->rodas_wg_f64, r->rodas_wg_f64_sv, r->wg_serve_init[0], r->wg_serve_tick[0]};
+        for (hipFunction_t fn : f64) {
+            int nb = 0;
+            if (fn && hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn, r->wg_threads[0], 0) == hipSuccess && nb < 1)
+                r->wg_threads[0] = 256;
+        }
     }
     return r;
 }
@@ -683,10 +703,6 @@ int ensure_ws(odemi_ctx* c, size_t bytes) {
     c->ws_bytes = b;
     return 0;
 }
-
-// Threads of the workgroup kernels: ODEMI_WG_THREADS, for the FP64 variant
-// ODEMI_WG_THREADS_F64 (kernels/odemi_wg.h).
-int wg_threads(int nmax, bool mixed) { return !mixed && nmax >= 96 ? 512 : 256; }
 
 // Row stride (and side) of each workgroup's FP32 Jacobian block in the mixed
 // workgroup kernels: 16 ceil(nmax / 16), as ODEMI_GJ_LD in kernels/odemi_gj.h.
@@ -832,7 +848,7 @@ int solve_impl(odemi_ctx* ctx, odemi_rhs* rhs, odemi_solve_args* a, bool noalloc
     const size_t vrows = plain_wg ? 3 : rodas ? (size_t)(3 + nmax) : 4;
     // ---- launch geometry of the persistent kernels ----
     const int block = a->block > 0 ? a->block : 256;
-    const int threads = use_wg ? wg_threads(nmax, mixed) : block;
+    const int threads = use_wg ? rhs->wg_threads[mixed ? 1 : 0] : block;
     const bool use_gj = use_wg && mixed && nmax <= 128;   // register-tiled Gauss-Jordan variant
     size_t shmem = 0;
     int64_t grid = 0;
@@ -862,7 +878,7 @@ int solve_impl(odemi_ctx* ctx, odemi_rhs* rhs, odemi_solve_args* a, bool noalloc
         shmem = wg_shmem_bytes(nmax, false, (rhs->features & 16) != 0, false);
         if (shmem > 160 * 1024) { ctx->err = "state dimension too large for the workgroup kernel's LDS"; return -3; }
         int nb = 0;
-        HIPCHK(ctx, hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn_main, wg_threads(nmax, false), shmem));
+        HIPCHK(ctx, hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn_main, rhs->wg_threads[0], shmem));
         grid = std::min<int64_t>((int64_t)std::max(nb, 1) * std::max(ctx->cu_count, 1), N);
     }
     // ---- workspace layout ----
@@ -1008,7 +1024,7 @@ int solve_impl(odemi_ctx* ctx, odemi_rhs* rhs, odemi_solve_args* a, bool noalloc
         const int lgrid = (int)((N + block - 1) / block);
         if (plain_wg) {
             // init: one workgroup per trajectory (grid-strided)
-            if (launch(ctx, fn_init, (int)grid, wg_threads(nmax, false), P, s, shmem)) return -1;
+            if (launch(ctx, fn_init, (int)grid, rhs->wg_threads[0], P, s, shmem)) return -1;
         } else {
             if (launch(ctx, fn_init, lgrid, block, P, s)) return -1;
         }
@@ -1021,7 +1037,7 @@ int solve_impl(odemi_ctx* ctx, odemi_rhs* rhs, odemi_solve_args* a, bool noalloc
             for (int k = 0; k < kBatch; k++) {
                 if (plain_wg) {
                     if (clear_words(ctx, P.counters, 2, s, true)) return -1;
-                    if (launch(ctx, fn_main, (int)grid, wg_threads(nmax, false), P, s, shmem)) return -1;
+                    if (launch(ctx, fn_main, (int)grid, rhs->wg_threads[0], P, s, shmem)) return -1;
                 } else {
                     if (k == kBatch - 1 && clear_words(ctx, P.counters + 1, 2, s, true)) return -1;
                     if (launch(ctx, fn_main, lgrid, block, P, s)) return -1;
@@ -1358,7 +1374,7 @@ extern "C" odemi_server* odemi_server_create(odemi_ctx* ctx, odemi_rhs* rhs, con
         S->shmem = wg_shmem_bytes(n, pi == 1, (rhs->features & 16) != 0, S->gj);   // dense rows for events
         if (S->shmem > 160 * 1024) { ctx->err = "state dimension too large for the workgroup kernel's LDS"; delete S; return nullptr; }
         int nb = 0;
-        if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&nb, rhs->wg_serve_tick[pi], wg_threads(n, pi == 1), S->shmem) != hipSuccess)
+        if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&nb, rhs->wg_serve_tick[pi], rhs->wg_threads[pi], S->shmem) != hipSuccess)
             nb = 1;
         S->wg_grid = std::max(nb, 1) * std::max(ctx->cu_count, 1);
     }
@@ -1663,7 +1679,7 @@ static void server_loop(odemi_server* S) {
                                  : (S->o.max_saves > 0 ? S->rhs->serve_tick_sv[S->o.alg][pi]
                                                        : S->rhs->serve_tick[S->o.alg][pi]);
     const size_t Sz = (size_t)S->S;
-    const unsigned wg_block = (unsigned)wg_threads(n, pi == 1);
+    const unsigned wg_block = (unsigned)S->rhs->wg_threads[pi];
     for (;;) {
         std::vector<Request*> admit;
         int64_t high = 0;
