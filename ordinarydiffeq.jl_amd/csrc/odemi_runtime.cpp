@@ -346,6 +346,39 @@ extern "C" void odemi_default_args(odemi_solve_args* a, int alg) {
     a->refine_sweeps = 1;
 }
 
+namespace {
+// Row stride (and side) of each workgroup's FP32 Jacobian block in the mixed
+// workgroup kernels: 16 ceil(nmax / 16), as ODEMI_GJ_LD in kernels/odemi_gj.h.
+size_t gj_ld(int nmax) { return 16 * (((size_t)nmax + 15) / 16); }
+
+// Dynamic LDS of the workgroup kernels; must match odemi::wg_layout in kernels/odemi_wg.h.
+size_t wg_shmem_bytes(int nmax, bool mixed, bool saves, bool gj) {
+    const size_t ld = (size_t)nmax | 1, fb = mixed ? 4 : 8;
+    const size_t np16 = 16 * (((size_t)nmax + 15) / 16);
+    size_t shmem = gj ? 0 : (((size_t)nmax * ld * fb + 15) & ~(size_t)15);
+    shmem += (size_t)(13 + (saves ? 3 : 0)) * nmax * 8 + 32 * 8;  // vectors + parameters (<= 32)
+    shmem += (size_t)(nmax + 32) * 4 + (size_t)nmax * 8;          // fsc + pf, piv + perm
+    shmem = (shmem + 15) & ~(size_t)15;
+    if (gj) shmem += 51 * np16 * 4;                        // Gauss-Jordan buffers + zbuf
+    shmem = (shmem + 15) & ~(size_t)15;
+    shmem += 32 * 8 + 32 * 4;
+    return shmem;
+}
+
+// Waves a SIMD that the FP64 workgroup kernels are compiled for (a cap on their
+// registers): as many workgroups of four waves as a CU's LDS holds, up to 4.
+// Left to itself the compiler takes 205 registers, two waves, and batches of
+// short chains, bound by latency, lose more by the missing workgroups than the
+// 55 spills of the cap at 4 cost (8,192 chains of n = 2..4: 31.1 -> 20.9 ms, of
+// 2..16: 43.2 -> 27.2, of 16..48: 85.2 -> 49.8; 300 chains, one workgroup a CU,
+// of 2..4: 3.2 -> 3.7, of 16..48: 9.7 -> 10.0; 5 and 6 are slower than 4
+// throughout).
+int wg_f64_waves(int n) {
+    const size_t lds = wg_shmem_bytes(n, false, false, false);
+    return (int)std::min<size_t>(4, 160 * 1024 / lds);
+}
+}  // namespace
+
 static std::string build_source(const char* problem_src, int n, int np, int flags) {
     std::ostringstream s;
     s << "#define ODEMI_N " << n << "\n#define ODEMI_NP " << (np > 0 ? np : 1) << "\n";
@@ -448,11 +481,12 @@ static std::string build_source(const char* problem_src, int n, int np, int flag
         // register cap for the mixed variant: minimum waves per SIMD (more
         // workgroups per CU against a few spills; 3 measured best at n = 128)
         const char* ww = getenv("ODEMI_WG_MIN_WAVES");
-        const int wgw = (ww && *ww) ? atoi(ww) : 3;
+        const int wgw = (ww && *ww) ? atoi(ww) : 3, wgw64 = wg_f64_waves(n);
         for (auto& k : v) {
             s << "extern \"C\" __global__ void __launch_bounds__("
               << (k[1][0] == 'f' ? "ODEMI_WG_THREADS" : "ODEMI_WG_THREADS_F64") << ") ";
-            if (wgw > 0 && k[1][0] == 'f') s << "__attribute__((amdgpu_waves_per_eu(" << wgw << "))) ";
+            const int w = k[1][0] == 'f' ? wgw : wgw64;
+            if (w > 1) s << "__attribute__((amdgpu_waves_per_eu(" << w << "))) ";
             s << k[0] << "(odemi::Params P) { odemi::rodas_wg_impl<" << k[1] << ", " << k[2] << ", " << k[3]
               << ">(P); }\n";
         }
@@ -463,7 +497,8 @@ static std::string build_source(const char* problem_src, int n, int np, int flag
         for (auto& k : sv) {
             s << "extern \"C\" __global__ void __launch_bounds__("
               << (k[2][0] == 'f' ? "ODEMI_WG_THREADS" : "ODEMI_WG_THREADS_F64") << ") ";
-            if (wgw > 0 && k[2][0] == 'f') s << "__attribute__((amdgpu_waves_per_eu(" << wgw << "))) ";
+            const int w = k[2][0] == 'f' ? wgw : wgw64;
+            if (w > 1) s << "__attribute__((amdgpu_waves_per_eu(" << w << "))) ";
             s << k[0] << "(odemi::Params P) { odemi::" << k[1] << "<" << k[2] << ", " << k[3] << ">(P); }\n";
         }
     }
@@ -702,24 +737,6 @@ int ensure_ws(odemi_ctx* c, size_t bytes) {
     HIPCHK(c, hipMalloc(&c->ws, b));
     c->ws_bytes = b;
     return 0;
-}
-
-// Row stride (and side) of each workgroup's FP32 Jacobian block in the mixed
-// workgroup kernels: 16 ceil(nmax / 16), as ODEMI_GJ_LD in kernels/odemi_gj.h.
-size_t gj_ld(int nmax) { return 16 * (((size_t)nmax + 15) / 16); }
-
-// Dynamic LDS of the workgroup kernels; must match odemi::wg_layout in kernels/odemi_wg.h.
-size_t wg_shmem_bytes(int nmax, bool mixed, bool saves, bool gj) {
-    const size_t ld = (size_t)nmax | 1, fb = mixed ? 4 : 8;
-    const size_t np16 = 16 * (((size_t)nmax + 15) / 16);
-    size_t shmem = gj ? 0 : (((size_t)nmax * ld * fb + 15) & ~(size_t)15);
-    shmem += (size_t)(13 + (saves ? 3 : 0)) * nmax * 8 + 32 * 8;  // vectors + parameters (<= 32)
-    shmem += (size_t)(nmax + 32) * 4 + (size_t)nmax * 8;          // fsc + pf, piv + perm
-    shmem = (shmem + 15) & ~(size_t)15;
-    if (gj) shmem += 51 * np16 * 4;                        // Gauss-Jordan buffers + zbuf
-    shmem = (shmem + 15) & ~(size_t)15;
-    shmem += 32 * 8 + 32 * 4;
-    return shmem;
 }
 
 int launch(odemi_ctx* c, hipFunction_t fn, int grid, int block, Params& P, hipStream_t s, size_t shmem = 0) {

@@ -100,3 +100,16 @@ def test_lost_copies_are_found():
     assert _lost(loop + [(8, "v_accvgpr_write_b32 a14, v212"), (16, "s_or_b64 exec, exec, s[0:1]")])
     assert not _lost(loop + [(8, "v_writelane_b32 v255, s10, 10"), (16, "s_or_b64 exec, exec, s[0:1]"),
                              (20, "v_mov_b32_e32 v1, v2")])
+
+
+def test_short_chains_share_a_compute_unit():
+    """Batches of short chains need four workgroups a CU: the FP64 kernels of
+    n = 16 take at most a quarter of a SIMD's registers."""
+    tr, _ = api.trace_for(P.CHAIN, 16, 3, algs=("rodas5p",), ns=[2, 16])
+    path, _ = _lib.precompile(tr.src, 16, 3, _lib.COMPILE_WG)
+    notes = subprocess.run([LLVM + "llvm-readelf", "--notes", path], capture_output=True, text=True, check=True).stdout
+    regs = dict((re.search(r"\.name:\s+(\S+)", k).group(1), int(re.search(r"\.vgpr_count:\s+(\d+)", k).group(1)))
+                for k in notes.split("- .agpr_count:")[1:])
+    assert all(4 * v <= 512 for k, v in regs.items() if "_f64" in k), regs
+    for name, code in _functions(path).items():
+        assert not _lost(code), (name, _lost(code))
