@@ -2502,6 +2502,12 @@ __device__ __forceinline__ int rodas_attempt(RodasLane<F, N>& L, const Params& P
 // v_readlane an attempt; here two scalar loads a stage, kept from being hoisted),
 // stage sums of the last stages that share their first five terms, and the
 // controller's rules.
+//
+// The sign of a zero stage value is not followed (add_tgrad leaves out a + 0,
+// the quotient of a -0 by a positive pivot comes out +0).  It reaches a state
+// only from a sum that begins with -0: the sums begin with uprev, go on from +0
+// where terms cancel, and no term a k underflows with the bound on the quotients
+// k below.  So an attempt from a state with a -0 is left to the complete rules.
 // ---------------------------------------------------------------------------
 
 // Dense LU on registers: the arithmetic of lu_factor_reg / lu_solve_reg.
@@ -2633,7 +2639,10 @@ __device__ __forceinline__ int rodas_attempt_fast(RodasLane<F, N>& L, FastCtl& F
     Ctl& c = L.c;
     const double left = c.tf - c.t;
     const double dt = fmin(fabs(FC.x), left);
-    if (!((dt > FC.bound) & (dt < 0x1p+450) & (dt > 0x1p-450) & (FC.att < itmax))) return -1;
+    bool neg0 = false;
+#pragma unroll
+    for (int i = 0; i < N; i++) neg0 = neg0 | __builtin_amdgcn_class(L.uprev[i], 0x20);
+    if (!((dt > FC.bound) & (dt < 0x1p+450) & (dt > 0x1p-450) & (FC.att < itmax)) | neg0) return -1;
     const bool last = !(dt + FC.tol < left);
     const double t = c.t;
     // 1/dt and 1/(dt gamma): rcp_nr for the mixed engine, the IEEE quotient for FP64
@@ -2721,7 +2730,8 @@ __device__ __forceinline__ int rodas_attempt_fast(RodasLane<F, N>& L, FastCtl& F
             pmax = fmax(pmax, fabs(LU.A[i][i]));
             pmin = fmin(pmin, fabs(LU.A[i][i]));
         }
-        ok = ok & (pmax < 0x1p+500) & (pmin > 0x1p-500) & (emin > -900);
+        ok = ok & (pmax < 0x1p+500) & (pmin > 0x1p-500) & (emin > -900) &
+             (emin - __builtin_amdgcn_frexp_exp(pmax) > -940);
     }
     const double EEst = fast_eest<HW, N>(s);
     float lg;
