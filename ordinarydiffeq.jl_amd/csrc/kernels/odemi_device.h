@@ -1723,7 +1723,8 @@ __device__ __forceinline__ void fast_init(FastCtl& F, const Ctl& c, const Params
     const double atf = fabs(c.tf);
     const bool regular = P.ntstops == 0 && P.abstol >= 0x1p-500 && P.abstol <= 0x1p+500 && P.reltol >= 0.0 &&
                          P.reltol <= 0.25 && fabs(P.dtmin) <= 0x1p+500 && c.tdir > 0.0 && atf >= 0x1p-500 &&
-                         atf <= 0x1p+500 && fabs(c.t) <= atf && c.dtmax <= 0x1p+600 && fabs(c.dt) <= 0x1p+600;
+                         atf <= 0x1p+500 && fabs(c.t) <= atf && c.dtmax <= 0x1p+600 && fabs(c.dt) <= 0x1p+600 &&
+                         (F.att > 0 || F.x >= 0.0);   // a first dt against tdir: the complete rules raise it
     const double e = jl_eps(atf);
     F.tol = 100.0 * e;
     F.bound = regular ? fmax(e, fabs(P.dtmin)) : __builtin_huge_val();

@@ -1,5 +1,6 @@
 """Edges of the lane kernels' common attempt against the complete rules: states
-that are a negative zero (compared by their bits).  A stopping time beyond every span sends each attempt
+that are a negative zero (compared by their bits), and a user dt against the
+direction of integration.  A stopping time beyond every span sends each attempt
 through the complete rules (see test_gpu_common_attempt.py)."""
 import numpy as np
 import pytest
@@ -94,3 +95,25 @@ def test_zero_states_bit_identical(alg, precision, fun, saveat):
     rows = np.arange(4)[:, None] < a["nsaved"][None, :]
     assert np.array_equal(_bits(np.swapaxes(a["u_out"], 1, 2)[rows]), _bits(np.swapaxes(b["u_out"], 1, 2)[rows]))
     assert (a["retcode"] == 1).mean() > 0.5
+
+@ALGS
+@PRECISIONS
+@pytest.mark.parametrize("dtmin", [0.0, 1e-3])
+def test_user_dt_against_the_direction(alg, precision, dtmin):
+    """The complete rules raise a negative dt of a forward solve to max(eps(t),
+    dtmin), where it ends (Unstable or DtLessThanMin)."""
+    u0, p, t0, tf = _batch(GROWTH, 200)
+    t0[::3] = 0.01
+    kw = dict(reltol=1e-6, abstol=1e-8, dt=-0.1, dtmin=dtmin, maxiters=500)
+    ea = odemi.EnsembleMI355X(precision=precision)
+    print(f"[case] negative dt {alg} {precision} dtmin {dtmin}", flush=True)
+    a = odemi.solve_arrays(GROWTH, alg, u0, p, t0, tf, ea, **kw)
+    b = odemi.solve_arrays(GROWTH, alg, u0, p, t0, tf, ea, tstops=[1e12], **kw)
+    outs = [b]
+    if precision == "fp64":
+        outs.append(odemi.solve_arrays(GROWTH, alg, u0, p, t0, tf, odemi.EnsembleMI355X(engine="plain"), **kw))
+    for o in outs:
+        assert np.array_equal(a["retcode"], o["retcode"]) and np.array_equal(a["stats"], o["stats"])
+        assert np.array_equal(a["u_final"], o["u_final"], equal_nan=True)
+        assert np.array_equal(a["t_final"], o["t_final"])
+    assert (a["retcode"] != 1).all()
