@@ -824,24 +824,6 @@ int solve_impl(odemi_ctx* ctx, odemi_rhs* rhs, odemi_solve_args* a, bool noalloc
         if (!plain) fn_prep = rhs->rodas_prep;
     }
     if (plain && mixed) { ctx->err = "the plain engine is FP64 only"; return -3; }
-    // Longest first only where the order matters.  Up to one workgroup of 256
-    // lanes per CU every lane takes one trajectory and every wave has its SIMD to
-    // itself: the solve lasts as long as its longest trajectory in any order, and
-    // the sort's three kernels, its fill and the records' unpacking are launches
-    // saved (1,024 Lorenz trajectories 277 -> 256 us a call; at 65,536 the longest
-    // wave is the same, above it waves share a SIMD and short ones should leave
-    // together).
-    const bool sorted = a->sort_by_cost && !plain && N > 0 &&
-                        ((rodas && (rhs->flags & ODEMI_COMPILE_WG)) || N > 256 * (int64_t)std::max(ctx->cu_count, 1));
-    // queue-order records (final-state-only Tsit5 persistent engine, no save
-    // before the end point, no lane callbacks; not in the allocation-free form;
-    // $ODEMI_QUEUE_RECORDS=0 reads and writes the SoA arrays in place instead)
-    const char* qr = getenv("ODEMI_QUEUE_RECORDS");
-    const bool use_rec = !(qr && atoi(qr) == 0) && !rodas && !plain && !noalloc && fn_prep && rhs->rec_unpack &&
-                         sorted &&
-                         a->nsaveat == 0 && !a->save_everystep && !a->save_start && !(rhs->features & 6) &&
-                         nmax == rhs->n;
-    const int rec_np = std::max(rhs->np, 1);
     if (!fn_main || (plain && !fn_init)) { ctx->err = "requested kernel was not compiled for this problem"; return -3; }
     if (a->nvec && !use_wg && !plain_wg) { ctx->err = "uneven batches (nvec) need the workgroup Rodas5P kernels"; return -3; }
     if ((use_wg || plain_wg) && (rhs->features & kLaneHooks)) {
@@ -898,6 +880,24 @@ int solve_impl(odemi_ctx* ctx, odemi_rhs* rhs, odemi_solve_args* a, bool noalloc
         HIPCHK(ctx, hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn_main, rhs->wg_threads[0], shmem));
         grid = std::min<int64_t>((int64_t)std::max(nb, 1) * std::max(ctx->cu_count, 1), N);
     }
+    // Longest first only where the order matters.  Where every lane of the launch
+    // takes one trajectory at most and every wave has its SIMD to itself (one
+    // workgroup of 256 lanes per CU), the solve lasts as long as its longest
+    // trajectory in any order, and the sort's three kernels, its fill and the
+    // records' unpacking are launches saved (1,024 Lorenz trajectories 277 -> 256
+    // us a call; at 65,536 the longest wave is the same, above it waves share a
+    // SIMD and short ones should leave together).
+    const bool sorted = a->sort_by_cost && !plain &&
+                        (use_wg || N > grid * threads || N > 256 * (int64_t)std::max(ctx->cu_count, 1));
+    // queue-order records (final-state-only Tsit5 persistent engine, no save
+    // before the end point, no lane callbacks; not in the allocation-free form;
+    // $ODEMI_QUEUE_RECORDS=0 reads and writes the SoA arrays in place instead)
+    const char* qr = getenv("ODEMI_QUEUE_RECORDS");
+    const bool use_rec = !(qr && atoi(qr) == 0) && !rodas && !plain && !noalloc && fn_prep && rhs->rec_unpack &&
+                         sorted &&
+                         a->nsaveat == 0 && !a->save_everystep && !a->save_start && !(rhs->features & 6) &&
+                         nmax == rhs->n;
+    const int rec_np = std::max(rhs->np, 1);
     // ---- workspace layout ----
     size_t need = 0;
     auto add = [&](size_t b) { need += ((b + 255) & ~size_t(255)); };
