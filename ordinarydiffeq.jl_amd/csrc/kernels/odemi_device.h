@@ -1714,18 +1714,21 @@ __device__ __forceinline__ void fast_to_ctl(const FastCtl& F, Ctl& c, const Para
     c.dt = c.tdir * ((F.att == 0) ? F.x : fabs(F.x));
     c.dtpropose = c.accept_step ? c.tdir * jl_max(F.x, fabs(jl_max(jl_eps(c.t), P.dtmin))) : c.dt;
 }
-// Once per trajectory (or serving tick), from a whole controller state.
 // Regular: forward, times of ordinary size with |t| <= |tf|, tolerances that
 // keep the error norm's denominators in range, no user stopping times.
+__device__ __forceinline__ bool fast_regular(const Params& P, double tdir, double t, double tf) {
+    const double atf = fabs(tf);
+    return P.ntstops == 0 && P.abstol >= 0x1p-500 && P.abstol <= 0x1p+500 && P.reltol >= 0.0 && P.reltol <= 0.25 &&
+           fabs(P.dtmin) <= 0x1p+500 && tdir > 0.0 && atf >= 0x1p-500 && atf <= 0x1p+500 && fabs(t) <= atf;
+}
+// Once per trajectory (or serving tick), from a whole controller state.  `leave`:
+// the state is one that the common attempt does not follow.
 template <bool SAVES>
-__device__ __forceinline__ void fast_init(FastCtl& F, const Ctl& c, const Params& P) {
+__device__ __forceinline__ void fast_init(FastCtl& F, const Ctl& c, const Params& P, bool leave = false) {
     fast_from_ctl(F, c);
-    const double atf = fabs(c.tf);
-    const bool regular = P.ntstops == 0 && P.abstol >= 0x1p-500 && P.abstol <= 0x1p+500 && P.reltol >= 0.0 &&
-                         P.reltol <= 0.25 && fabs(P.dtmin) <= 0x1p+500 && c.tdir > 0.0 && atf >= 0x1p-500 &&
-                         atf <= 0x1p+500 && fabs(c.t) <= atf && c.dtmax <= 0x1p+600 && fabs(c.dt) <= 0x1p+600 &&
+    const bool regular = !leave && fast_regular(P, c.tdir, c.t, c.tf) && c.dtmax <= 0x1p+600 && fabs(c.dt) <= 0x1p+600 &&
                          (F.att > 0 || F.x >= 0.0);   // a first dt against tdir: the complete rules raise it
-    const double e = jl_eps(atf);
+    const double e = jl_eps(fabs(c.tf));
     F.tol = 100.0 * e;
     F.bound = regular ? fmax(e, fabs(P.dtmin)) : __builtin_huge_val();
     if (regular && F.att == 0) F.x = fmin(F.x, c.dtmax);   // the first loop header's min(dtmax, dt)
@@ -1815,17 +1818,19 @@ __device__ __forceinline__ int tsit5_attempt_fast(Tsit5Lane<double, K, N>& L, Fa
     F.x = fmin(dtn, c.dtmax);
     return last ? RC_SUCCESS : 0;
 }
-// The same attempt by the complete rules.
-template <bool SAVES, typename K, int N>
-__device__ __forceinline__ int tsit5_attempt_full(Tsit5Lane<double, K, N>& L, FastCtl& F, const Params& P, i64 j) {
-    Ctl& c = L.c;
-    const int att0 = F.att;
-    fast_to_ctl(F, c, P);
-    if (c.accept_step) {
+// The state between attempts in its whole form, for an attempt by the complete
+// rules, and back.
+template <typename K, int N>
+__device__ __forceinline__ void tsit5_to_complete(Tsit5Lane<double, K, N>& L, const FastCtl& F, const Params& P) {
+    fast_to_ctl(F, L.c, P);
+    if (L.c.accept_step) {
 #pragma unroll
         for (int i = 0; i < N; i++) { L.u[i] = L.uprev[i]; L.k7[i] = L.k1[i]; }
     }
-    const int rc = tsit5_attempt<SAVES>(L, P, j);
+}
+template <bool SAVES, typename K, int N>
+__device__ __forceinline__ void tsit5_from_complete(Tsit5Lane<double, K, N>& L, FastCtl& F, const Params& P, int att0) {
+    Ctl& c = L.c;
     fast_from_ctl(F, c);
     c.nf -= 6 * (F.att - att0);
     if (c.accept_step) {
@@ -1833,6 +1838,14 @@ __device__ __forceinline__ int tsit5_attempt_full(Tsit5Lane<double, K, N>& L, Fa
         for (int i = 0; i < N; i++) { L.uprev[i] = L.u[i]; L.k1[i] = L.k7[i]; }
     }
     if (SAVES) fast_next_save(F, c, P);
+}
+// The same attempt by the complete rules.
+template <bool SAVES, typename K, int N>
+__device__ __forceinline__ int tsit5_attempt_full(Tsit5Lane<double, K, N>& L, FastCtl& F, const Params& P, i64 j) {
+    const int att0 = F.att;
+    tsit5_to_complete(L, F, P);
+    const int rc = tsit5_attempt<SAVES>(L, P, j);
+    tsit5_from_complete<SAVES>(L, F, P, att0);
     return rc;
 }
 // The counters that FastCtl::att stands for (c.nf holds the rest meanwhile).
@@ -1847,6 +1860,18 @@ constexpr bool kFastAttempts = false;
 #else
 constexpr bool kFastAttempts = true;
 #endif
+// For kernels with two loops, one with the common attempt and one without it: which
+// one a wave takes.  The first where most of a sample of the batch (its lanes'
+// trajectories in input order) is regular.  Both are right for every trajectory,
+// but in the first an irregular one pays for a check that fails and for two
+// changes of its state's form an attempt (100,003 Lorenz trajectories with save
+// times and a stopping time: FP64 2.77 ms in the first loop, 1.51 in the second).
+__device__ __forceinline__ bool fast_wave(const Params& P) {
+    const i64 k = (i64)blockIdx.x * blockDim.x + threadIdx.x, j = k < P.N ? k : P.N - 1;
+    const double t0 = P.t0[j], tf = P.tf[j];
+    const bool regular = fast_regular(P, (tf < t0) ? -1.0 : 1.0, t0, tf);
+    return 2 * __popcll(__ballot(regular)) > __popcll(__ballot(true));
+}
 __device__ __forceinline__ int fast_itmax(const Params& P) {
     return (int)(P.maxiters < 0x7fffffffLL ? P.maxiters : 0x7fffffffLL);
 }
@@ -1903,12 +1928,16 @@ __device__ __forceinline__ bool refill_now(bool need, bool active) {
     return need && (__popcll(needm) >= ODEMI_REFILL_MIN || __ballot(active) == 0);
 }
 
-template <bool SAVES, typename S, typename K, int N>
-__device__ void tsit5_persistent(const Params& P) {
+template <bool FAST, bool SAVES, typename S, typename K, int N>
+__device__ __forceinline__ void tsit5_persistent_loop(const Params& P) {
     Tsit5Lane<S, K, N> L;
     WaveQueue q;
     bool active = false, exhausted = false;
     i64 j = 0, js = 0;
+    // irregular lanes of the FAST loop keep their state in its whole form (DIRECT),
+    // or change it around every attempt, where there are no registers left for it
+    constexpr bool DIRECT = FAST && !SAVES && sizeof(K) < sizeof(S);
+    bool complete = false;
     FastCtl F;
     const int itmax = fast_itmax(P);
     (void)F; (void)itmax;
@@ -1920,9 +1949,10 @@ __device__ void tsit5_persistent(const Params& P) {
                 js = slot;
                 j = P.order ? P.order[slot] : slot;
                 tsit5_init(L, P, j, slot);
-                if constexpr (kFastAttempts) {
+                if constexpr (FAST) {
                     fast_init<SAVES>(F, L.c, P);
-                    L.c.nf -= 6 * F.att;
+                    complete = DIRECT && !(F.bound < __builtin_huge_val());
+                    if (!complete) L.c.nf -= 6 * F.att;
                 }
                 active = true;
             } else {
@@ -1932,22 +1962,45 @@ __device__ void tsit5_persistent(const Params& P) {
         if (__ballot(active) == 0) break;
         if (active) {
             int rc;
-            if constexpr (kFastAttempts) {
-                // until a lane of the wave ends
-                do rc = tsit5_attempt_fast<SAVES>(L, F, P, j, itmax);
-                while (__ballot(rc != 0) == 0);
-                if (__builtin_expect(rc < 0, 0)) rc = tsit5_attempt_full<SAVES>(L, F, P, j);
+            if constexpr (FAST) {
+                rc = -1;
+                if (!complete) {   // until a lane of the wave ends
+                    do rc = tsit5_attempt_fast<SAVES>(L, F, P, j, itmax);
+                    while (__ballot(rc != 0) == 0);
+                }
+                if (__builtin_expect(rc < 0, 0)) {
+                    const int att0 = F.att;
+                    if (!complete) tsit5_to_complete(L, F, P);
+                    rc = tsit5_attempt<SAVES>(L, P, j);
+                    if (!complete) tsit5_from_complete<SAVES>(L, F, P, att0);
+                }
             } else {
                 rc = tsit5_attempt<SAVES>(L, P, j);
             }
             if (rc) {
-                if constexpr (kFastAttempts) fast_counts(F, L.c);
+                if (FAST && !complete) fast_counts(F, L.c);
                 if (!SAVES && P.rec_out) finish_lane_rec<N>(L.c, P, js, L.u, rc);
                 else finish_lane<N>(L.c, P, j, L.u, rc);
                 active = false;
             }
         }
     }
+}
+// The saving kernels hold both loops.  In the others a second loop costs the first
+// (FP64: 16 reloads of spilled scalar registers an attempt, 1M Lorenz trajectories
+// 2.23 -> 2.30 ms; mixed: 300,007 trajectories 0.64 -> 0.68 ms), so there it is a
+// kernel of its own (COMPLETE), which the host takes where the options make every
+// trajectory irregular or it sees backward spans; those in device arrays stay in
+// the first.
+template <bool SAVES, typename S, typename K, int N, bool COMPLETE = false>
+__device__ void tsit5_persistent(const Params& P) {
+    if constexpr (kFastAttempts && SAVES) {
+        if (!fast_wave(P)) {
+            tsit5_persistent_loop<false, SAVES, S, K, N>(P);
+            return;
+        }
+    }
+    tsit5_persistent_loop<kFastAttempts && !COMPLETE, SAVES, S, K, N>(P);
 }
 
 // Plain engine: one kernel launch per step attempt, state in HBM.
@@ -2508,7 +2561,9 @@ __device__ __forceinline__ int rodas_attempt(RodasLane<F, N>& L, const Params& P
 // the quotient of a -0 by a positive pivot comes out +0).  It reaches a state
 // only from a sum that begins with -0: the sums begin with uprev, go on from +0
 // where terms cancel, and no term a k underflows with the bound on the quotients
-// k below.  So an attempt from a state with a -0 is left to the complete rules.
+// k below.  So a trajectory is left to the complete rules from where its state
+// has a -0 (at its start, or after an attempt by those; a common attempt never
+// ends in one).
 // ---------------------------------------------------------------------------
 
 // Dense LU on registers: the arithmetic of lu_factor_reg / lu_solve_reg.
@@ -2640,10 +2695,7 @@ __device__ __forceinline__ int rodas_attempt_fast(RodasLane<F, N>& L, FastCtl& F
     Ctl& c = L.c;
     const double left = c.tf - c.t;
     const double dt = fmin(fabs(FC.x), left);
-    bool neg0 = false;
-#pragma unroll
-    for (int i = 0; i < N; i++) neg0 = neg0 | __builtin_amdgcn_class(L.uprev[i], 0x20);
-    if (!((dt > FC.bound) & (dt < 0x1p+450) & (dt > 0x1p-450) & (FC.att < itmax)) | neg0) return -1;
+    if (!((dt > FC.bound) & (dt < 0x1p+450) & (dt > 0x1p-450) & (FC.att < itmax))) return -1;
     const bool last = !(dt + FC.tol < left);
     const double t = c.t;
     // 1/dt and 1/(dt gamma): rcp_nr for the mixed engine, the IEEE quotient for FP64
@@ -2724,15 +2776,14 @@ __device__ __forceinline__ int rodas_attempt_fast(RodasLane<F, N>& L, FastCtl& F
     const double s = fast_error_sum<N>(ks[7], L.uprev, L.u, P.abstol, P.reltol);
     bool ok = s < 0x1p+1000;
     if constexpr (!HW) {
-        // the pivots' and dividends' range for the quotients
+        // the pivots' and dividends' range for the quotients, none below 2^-941 but 0
         double pmax = fabs(LU.A[0][0]), pmin = pmax;
 #pragma unroll
         for (int i = 1; i < N; i++) {
             pmax = fmax(pmax, fabs(LU.A[i][i]));
             pmin = fmin(pmin, fabs(LU.A[i][i]));
         }
-        ok = ok & (pmax < 0x1p+500) & (pmin > 0x1p-500) & (emin > -900) &
-             (emin - __builtin_amdgcn_frexp_exp(pmax) > -940);
+        ok = ok & (pmax < 0x1p+100) & (pmin > 0x1p-500) & (emin > -840);
     }
     const double EEst = fast_eest<HW, N>(s);
     float lg;
@@ -2782,6 +2833,13 @@ __device__ __forceinline__ void rodas_fast_counts(const FastCtl& F, Ctl& c, int 
     c.nw += sign * F.att;
     c.nsolve += sign * 8 * F.att;
 }
+template <int N>
+__device__ __forceinline__ bool neg_zero(const double (&u)[N]) {
+    bool z = false;
+#pragma unroll
+    for (int i = 0; i < N; i++) z = z | __builtin_amdgcn_class(u[i], 0x20);
+    return z;
+}
 // The same attempt by the complete rules.
 template <typename F, int N>
 __device__ __forceinline__ int rodas_attempt_full(RodasLane<F, N>& L, FastCtl& FC, const Params& P, i64 j) {
@@ -2807,11 +2865,12 @@ __device__ __forceinline__ int rodas_attempt_full(RodasLane<F, N>& L, FastCtl& F
         for (int i = 0; i < N; i++) L.uprev[i] = L.u[i];
     }
     fast_next_save(FC, c, P);
+    FC.bound = neg_zero(L.uprev) ? __builtin_huge_val() : FC.bound;
     return rc;
 }
 
-template <typename F, int N>
-__device__ void rodas_persistent(const Params& P) {
+template <bool FAST, typename F, int N>
+__device__ __forceinline__ void rodas_persistent_loop(const Params& P) {
     RodasLane<F, N> L;
     WaveQueue q;
     bool active = false, exhausted = false;
@@ -2826,8 +2885,8 @@ __device__ void rodas_persistent(const Params& P) {
             if (slot < P.N) {
                 j = P.order ? P.order[slot] : slot;
                 rodas_init(L, P, j);
-                if constexpr (kFastAttempts) {
-                    fast_init<true>(FC, L.c, P);
+                if constexpr (FAST) {
+                    fast_init<true>(FC, L.c, P, neg_zero(L.uprev));
                     rodas_fast_counts(FC, L.c, -1);
                 }
                 active = true;
@@ -2838,7 +2897,7 @@ __device__ void rodas_persistent(const Params& P) {
         if (__ballot(active) == 0) break;
         if (active) {
             int rc;
-            if constexpr (kFastAttempts) {
+            if constexpr (FAST) {
                 // until a lane of the wave ends
                 do rc = rodas_attempt_fast(L, FC, P, j, itmax);
                 while (__ballot(rc != 0) == 0);
@@ -2847,12 +2906,28 @@ __device__ void rodas_persistent(const Params& P) {
                 rc = rodas_attempt(L, P, j);
             }
             if (rc) {
-                if constexpr (kFastAttempts) rodas_fast_counts(FC, L.c, 1);
+                if constexpr (FAST) rodas_fast_counts(FC, L.c, 1);
                 finish_lane<N>(L.c, P, j, L.u, rc);
                 active = false;
             }
         }
     }
+}
+// The FP64 kernel has the one loop only: a second one would cost regular batches
+// 2 % (262,144 Robertson trajectories 1.26 -> 1.29 ms), and irregular ones stay
+// near what the complete rules alone took (two stopping times 2.5-2.9 ms from run
+// to run, 2.66 then).  Mixed: two stopping times 2.09 -> 1.89 ms, regular ones the
+// same.
+template <typename F, int N>
+__device__ void rodas_persistent(const Params& P) {
+    constexpr bool two = kFastAttempts && sizeof(F) < sizeof(double);
+    if constexpr (two) {
+        if (!fast_wave(P)) {
+            rodas_persistent_loop<false, F, N>(P);
+            return;
+        }
+    }
+    rodas_persistent_loop<kFastAttempts, F, N>(P);
 }
 
 // Plain Rodas5P: st_vec rows u, uprev, dT, J[0..N-1]
@@ -3063,7 +3138,7 @@ __device__ void rodas_serve_tick(const Params& P0) {
 #pragma unroll
             for (int i = 0; i < N; i++) L.uprev[i] = L.u[i];
         }
-        fast_init<true>(FC, L.c, P);
+        fast_init<true>(FC, L.c, P, neg_zero(L.uprev));
         rodas_fast_counts(FC, L.c, -1);
     }
     for (int a = 0; a < P.tick_attempts; a++) {

@@ -13,6 +13,7 @@
 #include <hip/hiprtc.h>
 
 #include <algorithm>
+#include <cmath>
 #include <chrono>
 #include <cstdio>
 #include <cstdlib>
@@ -266,6 +267,7 @@ struct odemi_rhs {
     int wg_threads[2] = {256, 256};   // of the workgroup kernels [fp64, mixed]
     int features = 0;   // lane hooks 1 isoutofdomain, 2 discrete, 4 continuous callbacks; workgroup callbacks 8, 16
     hipFunction_t tsit5_persist_f64 = nullptr, tsit5_persist_mixed = nullptr;
+    hipFunction_t tsit5_persist_complete[2] = {};   // by the complete rules alone [fp64, mixed]
     hipFunction_t tsit5_persist_f64_sv = nullptr, tsit5_persist_mixed_sv = nullptr;
     hipFunction_t tsit5_plain_init = nullptr, tsit5_plain_step = nullptr;
     hipFunction_t rodas_persist_f64 = nullptr, rodas_persist_mixed = nullptr;
@@ -409,6 +411,10 @@ static std::string build_source(const char* problem_src, int n, int np, int flag
     // engine: 1.91 -> 1.76 ms)
     s << "#ifndef ODEMI_MIN_WAVES\n#ifdef ODEMI_NCCB\n#define ODEMI_MIN_WAVES 3\n#else\n"
          "#define ODEMI_MIN_WAVES 4\n#endif\n#endif\n";
+    // the saving variants hold the dense output beside the attempt: 3 waves (at 4
+    // they spill up to 147 registers; 100,003 Lorenz trajectories with 20 save times
+    // 1.27 -> 1.02 ms, with a stopping time too 2.48 -> 1.51 ms)
+    s << "#define ODEMI_MIN_WAVES_SV (ODEMI_MIN_WAVES < 3 ? ODEMI_MIN_WAVES : 3)\n";
     s << kDeviceSource << "\n";
     // layout check of the kernel argument struct against this file's mirror
     s << "extern \"C\" __device__ const unsigned odemi_params_bytes = sizeof(odemi::Params);\n";
@@ -424,9 +430,17 @@ static std::string build_source(const char* problem_src, int n, int np, int flag
                                {"odemi_tsit5_persist_mixed", "false", "float"},
                                {"odemi_tsit5_persist_mixed_sv", "true", "float"}};
         for (auto& k : v)
-            s << "extern \"C\" __global__ void __launch_bounds__(256, ODEMI_MIN_WAVES) " << k[0]
+            s << "extern \"C\" __global__ void __launch_bounds__(256, "
+              << (k[1][0] == 't' ? "ODEMI_MIN_WAVES_SV" : "ODEMI_MIN_WAVES") << ") " << k[0]
               << "(odemi::Params P) { odemi::tsit5_persistent<" << k[1] << ", double, " << k[2]
               << ", ODEMI_N>(P); }\n";
+        // modules without common attempts (user hooks) have the complete rules in the first kernel
+        s << "#if !defined(ODEMI_NDCB) && !defined(ODEMI_NCCB) && !defined(ODEMI_HAS_ISOUT)\n";
+        for (const char* k : {"f64", "mixed"})
+            s << "extern \"C\" __global__ void __launch_bounds__(256, ODEMI_MIN_WAVES) odemi_tsit5_persist_" << k
+              << "_complete(odemi::Params P) { odemi::tsit5_persistent<false, double, " << (k[0] == 'f' ? "double" : "float")
+              << ", ODEMI_N, true>(P); }\n";
+        s << "#endif\n";
         s << "extern \"C\" __global__ void __launch_bounds__(256) odemi_tsit5_plain_init(odemi::Params P)"
              " { odemi::tsit5_plain_init<ODEMI_N>(P); }\n";
         s << "extern \"C\" __global__ void __launch_bounds__(256) odemi_tsit5_prep_f64(odemi::Params P)"
@@ -647,6 +661,10 @@ extern "C" odemi_rhs* odemi_compile_rhs(odemi_ctx* ctx, const char* problem_src,
     };
     if (flags & ODEMI_COMPILE_TSIT5) {
         get("odemi_tsit5_persist_f64", &r->tsit5_persist_f64);
+        if (!(r->features & kLaneHooks)) {
+            get("odemi_tsit5_persist_f64_complete", &r->tsit5_persist_complete[0]);
+            get("odemi_tsit5_persist_mixed_complete", &r->tsit5_persist_complete[1]);
+        }
         get("odemi_tsit5_persist_mixed", &r->tsit5_persist_mixed);
         get("odemi_tsit5_persist_f64_sv", &r->tsit5_persist_f64_sv);
         get("odemi_tsit5_persist_mixed_sv", &r->tsit5_persist_mixed_sv);
@@ -807,7 +825,27 @@ int solve_impl(odemi_ctx* ctx, odemi_rhs* rhs, odemi_solve_args* a, bool noalloc
         if (plain) { fn_init = rhs->tsit5_plain_init; fn_main = rhs->tsit5_plain_step; }
         else if (a->nsaveat > 0 || a->save_everystep)
             fn_main = mixed ? rhs->tsit5_persist_mixed_sv : rhs->tsit5_persist_f64_sv;
-        else fn_main = mixed ? rhs->tsit5_persist_mixed : rhs->tsit5_persist_f64;
+        else {
+            // Options with which no trajectory makes common attempts (fast_regular in
+            // kernels/odemi_device.h; either kernel is right for any): 1M Lorenz
+            // trajectories with two stopping times FP64 3.99 -> 3.17 ms, mixed 2.81 ->
+            // 2.36, with abstol 0 3.97 -> 3.14 and 2.75 -> 2.33.  And, in host arrays,
+            // mostly backward spans, by a sample (half a million over 0.1..0.4, FP64:
+            // 1.35 in the first kernel, 1.13 here; mixed 0.85 and 0.82).
+            bool common = a->ntstops == 0 && a->abstol >= 0x1p-500 && a->abstol <= 0x1p+500 && a->reltol >= 0.0 &&
+                          a->reltol <= 0.25 && std::fabs(a->dtmin) <= 0x1p+500;
+            if (common && !a->device_ptrs) {
+                const int64_t m = std::min<int64_t>(N, 64);
+                int64_t back = 0;
+                for (int64_t k = 0; k < m; k++) {
+                    const int64_t j = k * (N / m);
+                    back += a->tf[j] < a->t0[j] ? 1 : 0;
+                }
+                common = 2 * back <= m;
+            }
+            const hipFunction_t complete = common ? nullptr : rhs->tsit5_persist_complete[mixed ? 1 : 0];
+            fn_main = complete ? complete : mixed ? rhs->tsit5_persist_mixed : rhs->tsit5_persist_f64;
+        }
         if (!plain) fn_prep = rhs->tsit5_prep[mixed ? 1 : 0];
     } else if (plain_wg) {
         fn_init = rhs->wg_serve_init[0]; fn_main = rhs->wg_serve_tick[0];
