@@ -20,8 +20,6 @@ __device__ __forceinline__ void odemi_tgrad(T* __restrict__ dT, const T* __restr
     dT[0] = T(0); dT[1] = T(0); dT[2] = T(0);
 }
 #include "odemi_device.h"
-#include "odemi_gj.h"
-#include "odemi_lu.h"
 extern "C" __global__ void __launch_bounds__(256) k1(odemi::Params P) { odemi::tsit5_persistent<false, double, double, 3>(P); }
 extern "C" __global__ void __launch_bounds__(256) k2(odemi::Params P) { odemi::tsit5_persistent<false, double, float, 3>(P); }
 extern "C" __global__ void __launch_bounds__(256) k3(odemi::Params P) { odemi::tsit5_plain_init<3>(P); }
@@ -30,17 +28,3 @@ extern "C" __global__ void __launch_bounds__(256) k5(odemi::Params P) { odemi::r
 extern "C" __global__ void __launch_bounds__(256) k6(odemi::Params P) { odemi::rodas_persistent<float, 3>(P); }
 extern "C" __global__ void __launch_bounds__(256) k7(odemi::Params P) { odemi::rodas_plain_init<3>(P); }
 extern "C" __global__ void __launch_bounds__(256) k8(odemi::Params P) { odemi::rodas_plain_step<3>(P); }
-extern "C" __global__ void __launch_bounds__(256) lu_check(const double* A, int n, double* x) {
-    extern __shared__ double sh[];   // W [n][n | 1], right-hand side [n], then three int arrays
-    const int ld = n | 1;
-    double* b = sh + n * ld;
-    int* perm = (int*)(b + n);
-    for (int e = threadIdx.x; e < n * n; e += blockDim.x) sh[(e / n) * ld + e % n] = A[e];
-    for (int i = threadIdx.x; i < n; i += blockDim.x) b[i] = x[i];
-    __syncthreads();
-    odemi::wg_lu_blocked<2>(sh, ld, n, (int*)(((size_t)(perm + n) + 15) & ~(size_t)15), perm);
-    if (threadIdx.x < 64 && !odemi::wave_lu_solve<2, false>(sh, ld, n, perm, b))
-        for (int i = threadIdx.x; i < n; i += 64) b[i] = __builtin_nan("");
-    __syncthreads();
-    for (int i = threadIdx.x; i < n; i += blockDim.x) x[i] = b[i];
-}
