@@ -230,9 +230,9 @@ constexpr double kLN10 = 2.302585092994046, kLN2 = 0.6931471805599453;
 
 // FastPower.jl 1.1.x `fastpower` (controllers.jl:815-816): Goldberg's rational
 // fast log2 in Float32, then exp2 of the Float32 product, rounded once to
-// Float32.  The significand after the select lies in [-1/2, 1/2), so the
+// Float32.  The significand after the select lies in [-1/4, 1/2), so the
 // rational's quotient needs no scaling: v_rcp_f32, one Newton step and one
-// residual correction give the IEEE quotient for each of the 2^24 significands.
+// residual correction give the IEEE quotient for each of its 2^23 values.
 __device__ __forceinline__ float fastlog2f(float x) {
     const unsigned ux1i = __float_as_uint(x);
     const unsigned ex = (ux1i & 0x7F800000u) >> 23;

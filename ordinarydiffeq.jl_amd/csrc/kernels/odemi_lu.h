@@ -1,6 +1,6 @@
 // odemi_lu.h -- FP64 LU with partial pivoting of a matrix in LDS, factored by
-// the 256-thread workgroup of the FP64 workgroup Rodas5P kernels, and the
-// triangular solves with it.
+// the workgroup of the FP64 Rodas5P kernels (256 threads, or 512 where they are
+// built for eight waves), and the triangular solves with it.
 //
 // Every element sees the fma sequence of the sequential right-looking LU
 // (a_ij -= l_ik u_kj, k ascending) and of the column-ordered substitutions, and
@@ -9,9 +9,11 @@
 //
 // Bound: the instruction latency of one wave (a chain of 2 n substitution steps
 // a solve, n pivot steps a factorization), one trajectory a workgroup.  Measured
-// alone on a CU at n = 128: factorization ~60 us (85,000 cycles of it in the
-// panels), solve 8 us; 96 chains of n = 8..128 together 43.2 -> 10.0 ms against
-// the element-by-element factorization and IEEE quotients in every step.
+// with these functions alone, one workgroup a CU: factorization 84 us with four
+// waves, 79 us with eight at n = 128 (53 and 50 at 96, 28 and 27 at 64, 12 at 32);
+// solve, one wave in both, 8.2 us (6.4, 4.4, 2.5).  96 chains of n = 8..128 with
+// the element-by-element factorization and IEEE quotients in every step 43.2 ms,
+// with this one 10.5 ms on four waves and 10.0 ms on eight from n = 96 on.
 #pragma once
 
 namespace odemi {

@@ -13,7 +13,8 @@
 //   vec  double[NV][nmax]                 u, uprev, fsal, du, dT, ks[8] (+ dense[3]);
 //   pd   double[32]                       parameters (FP64)
 //   fsc  float[nmax + 32]                 FP32 copies of uprev and p (mixed variant)
-//   piv  int[nmax], perm int[nmax]        row positions (scratch of the LU) and the row gather
+//   piv  int[nmax], perm int[nmax]        row positions (scratch of the FP32 LU; the FP64 one
+//                                         uses ired) and the row gather
 //   gjbuf float[51 NP]                    Gauss-Jordan panels, pivot rows, scales and
 //                                         mat-vec result (mixed variant; NP = 16 R,
 //                                         R = ceil(nmax/16); layout in odemi_gj.h)
