@@ -1,5 +1,5 @@
 // The FP64 LU and substitutions of the workgroup kernels by themselves, for
-// tests/test_gpu_lu_check.py: lu_check factors and solves one matrix a workgroup.
+// tests/test_gpu_wg_lu_check.py: lu_check factors and solves one matrix a workgroup.
 // Built once for each number of row slots (ODEMI_N = 64, 128, 135: as large as a
 // CU's LDS holds); launched with 256 or 512 threads.
 #include <hip/hip_runtime.h>
